@@ -27,6 +27,7 @@ SOURCES = [
     CSRC / "prefill_attn.hip",
     CSRC / "copy_pages.hip",
     CSRC / "linear.hip",
+    CSRC / "gemm.hip",
     CSRC / "static_scratch.hip",
     CSRC / "sampling.hip",
     CSRC / "host" / "kvcache" / "block_manager.cpp",
@@ -69,8 +70,9 @@ def common_flags() -> list[str]:
 
 
 # Per-source additions. The decode kernel rescales its MFMA accumulators on the
-# VALU every page: they stay in VGPRs (the VGPR form of v_mfma) instead of
-# being copied out of and back into AGPRs around each rescale. Its first seven
+# VALU every page, and the prompts' linear layers add theirs up there run by run:
+# they stay in VGPRs (the VGPR form of v_mfma) instead of being copied out of and
+# back into AGPRs around each rescale or sum. Its first seven
 # kernel arguments (the work descriptors' address, n_kv, the pools, the block
 # tables, qkv and the rotary frequencies) are preloaded into scalar registers at
 # launch, so a work-group's descriptor load does not wait for a kernel-argument
@@ -82,6 +84,7 @@ def common_flags() -> list[str]:
 EXTRA_FLAGS = {
     "paged_decode.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-amdgpu-kernarg-preload-count=7"],
     "linear.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=9"],
+    "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "kv_append.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=8"],
     "prefill_attn.hip": ["-mllvm", "-amdgpu-kernarg-preload-count=9"],
 }

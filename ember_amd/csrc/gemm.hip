@@ -1,0 +1,348 @@
+// The linear layers of a prompt on gfx950: C[M, N] = A[M, K] . W[N, K]^T for
+// more rows than the decode-sized kernel takes (linear.hip, 64), with the same
+// four epilogues and the same bits per row (linear.hpp: the order of the sums).
+//
+// What bounds it: the matrix cores, once W and A are re-read little enough; at
+// few tokens, one work-group's chain of chunks. A work-group of 4 waves covers
+// 64 tokens x 64 FW features; each wave owns 16 FW features and all the tokens.
+// So W, packed in the MFMA operand's lane order, goes straight from memory to
+// registers, every wave its own, and only A passes through LDS, where each wave
+// reads it. A comes in chunks of two k steps, double-buffered, its loads two
+// chunks ahead in registers; W's loads run two chunks ahead too. Taking a run's
+// strided steps one at a time would read A in 64-byte pieces (1800 x 4096 x
+// 1024 29.1 us); two runs side by side read 128.
+//
+// Measured (packed W, a graph of 60 launches over 8 weights), against 64 rows
+// per launch of the decode-sized kernel: 1800 x 4096 x 1024 26.4 us (572
+// TFLOP/s), 129 before; 1800 x 1024 x 2048 17.8, 122; 1800 x 6144 x 1024 40.3,
+// 233; 1800 x 1024 x 3072 23.1, 166; 256 x 4096 x 1024 8.3, 19.8; 256 x 1024 x
+// 2048 11.9, 17.2. A 1800-token prompt of the 28-layer model: 19.93 -> 4.86 ms.
+#include <algorithm>
+#include <type_traits>
+
+#include "linear.hpp"
+
+namespace ember::hip {
+namespace {
+
+constexpr int kGemmWaves = 4;
+constexpr int kGemmThreads = kGemmWaves * kWave;
+constexpr int MT = 4;  // 16-token tiles per work-group
+constexpr int CS = 2;  // k steps per LDS chunk of A
+constexpr int kXcds = 8;
+constexpr int kDescWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
+
+// SLICES: K is split in KS slices as the decode-sized kernel splits this shape.
+template <int FW, int EP, bool SLICES, bool RAGGED>
+__global__ void __launch_bounds__(kGemmThreads, 2)
+    gemm_kernel(const f16 *__restrict__ A, int lda, const f16 *__restrict__ W, int M, int N, int K,
+                void *__restrict__ C, int ldc, int n_blocks, int slice_steps) {
+    constexpr int kRows = 16 * MT;
+    constexpr int kPieces = CS * 4;  // 16-byte pieces of a row per chunk of CS k steps
+    constexpr int kSwizzle = kPieces < 16 ? kPieces - 1 : 15;
+    constexpr int kLoads = kRows * kPieces / kGemmThreads;  // 16-byte pieces of A per thread and chunk
+    static_assert(kRows * kPieces % kGemmThreads == 0 && (CS & (CS - 1)) == 0);
+    __shared__ __align__(16) unsigned char lds[2][kRows * kPieces * 16];
+    const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int c = lane % 16, g = lane / 16;
+    // Block id -> (token block, feature block). Ids that differ by a multiple
+    // of 8 run on one XCD: with feature blocks in multiples of 8, an XCD takes
+    // an eighth of them for every token block, so its L2 keeps that part of W.
+    int mb, nb;
+    const int id = static_cast<int>(blockIdx.x);
+    if (n_blocks % kXcds == 0) {
+        const int per = n_blocks / kXcds, i = id / kXcds;
+        nb = (id % kXcds) * per + i % per;
+        mb = i / per;
+    } else {
+        nb = id % n_blocks;
+        mb = id / n_blocks;
+    }
+    const int m0 = mb * kRows, rows = min(M - m0, kRows);
+    const int steps = K / 32;
+    const int tiles = (N + 15) / 16, t0 = (nb * kGemmWaves + wave) * FW;
+
+    // A through a descriptor of this block's rows: rows past M (and the last
+    // chunk's columns past the last row's end) read as zeros.
+    const f16 *a0 = A + static_cast<int64_t>(m0) * lda;
+    const uint32_t records = static_cast<uint32_t>((static_cast<int64_t>(rows - 1) * lda + K) * 2);
+    const __amdgpu_buffer_rsrc_t ad = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16 *>(a0), 0, records, kDescWord3);
+    uint32_t aoff[kLoads];  // byte offset of this thread's pieces at k step 0
+    int aslot[kLoads];      // and their place in LDS: piece q of row r at slot kPieces r + (q ^ (r & kSwizzle))
+#pragma unroll
+    for (int j = 0; j < kLoads; j++) {
+        const int p = tid + j * kGemmThreads, r = p / kPieces, q = p % kPieces;
+        aoff[j] = r < rows ? static_cast<uint32_t>(r * lda + 8 * q) * 2u : records;
+        aslot[j] = 16 * (r * kPieces + (q ^ (r & kSwizzle)));
+    }
+    const f16 *w[FW];
+#pragma unroll
+    for (int f = 0; f < FW; f++)
+        w[f] = W + static_cast<int64_t>(min(t0 + f, tiles - 1)) * steps * kPackBlock + 8 * lane;
+
+    // A chunk is two adjacent k steps (128 bytes of a row of A). Unsplit, they
+    // belong to runs 2 p and 2 p + 1, which are summed side by side: chunks 2 p,
+    // 2 p + 8, ..., then the next pair of runs. In a slice they follow each
+    // other in one run. next_chunk(b): the chunk after the one at step b (S: none).
+    auto next_chunk = [&](int b) {
+        if (SLICES) return b + 2;
+        return b + kLinearRuns < steps ? b + kLinearRuns
+               : b < steps && b % kLinearRuns + 2 < min(kLinearRuns, steps) ? b % kLinearRuns + 2
+                                                                            : steps;
+    };
+    int a_chunk = 0;  // the chunk that load_a takes next
+    auto load_a = [&](uint4 (&v)[kLoads]) {
+        const uint32_t k = 64u * static_cast<uint32_t>(a_chunk);
+        a_chunk = next_chunk(a_chunk);
+#pragma unroll
+        for (int j = 0; j < kLoads; j++)  // an offset at or past the records reads zeros
+            v[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ad, min(aoff[j] + k, records), 0, 0));
+    };
+    auto store_a = [&](int buf, const uint4 (&v)[kLoads]) {
+#pragma unroll
+        for (int j = 0; j < kLoads; j++) *reinterpret_cast<uint4 *>(lds[buf] + aslot[j]) = v[j];
+    };
+    int w_chunk = 0;  // the chunk whose W goes out next
+    auto load_w = [&](int v, f16x8 (&wv)[FW]) {
+        const int64_t at = static_cast<int64_t>(min(w_chunk + v, steps - 1)) * kPackBlock;
+        if (v == CS - 1) w_chunk = next_chunk(w_chunk);
+#pragma unroll
+        for (int f = 0; f < FW; f++) wv[f] = *reinterpret_cast<const f16x8 *>(w[f] + at);
+    };
+
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int kAccs = SLICES ? 1 : 2;  // runs summed side by side
+    f32x4 acc[kAccs][FW][MT], sum[FW][MT], total[SLICES ? FW : 1][SLICES ? MT : 1];
+#pragma unroll
+    for (int f = 0; f < FW; f++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int r = 0; r < kAccs; r++) acc[r][f][mt] = zero;
+            sum[f][mt] = zero;
+            if constexpr (SLICES) total[f][mt] = zero;
+        }
+    // The MFMAs of a chunk's k step v: every tile of the wave, from zero at the start of a run.
+    auto mfmas = [&](auto first, int v, const f16x8 (&x)[MT], const f16x8 (&wv)[FW]) {
+        f32x4(&ac)[FW][MT] = acc[SLICES ? 0 : v];
+#pragma unroll
+        for (int f = 0; f < FW; f++)
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+                ac[f][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[f], x[mt], decltype(first)::value ? zero : ac[f][mt],
+                                                                   0, 0, 0);
+    };
+    auto end_runs = [&]() {  // the runs' sums join the slice's
+#pragma unroll
+        for (int r = 0; r < kAccs; r++)
+#pragma unroll
+            for (int f = 0; f < FW; f++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) sum[f][mt] = sum[f][mt] + acc[r][f][mt];
+    };
+    auto end_slice = [&]() {  // the slice's sum joins the total
+        if constexpr (SLICES) {
+#pragma unroll
+            for (int f = 0; f < FW; f++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+                    total[f][mt] = total[f][mt] + sum[f][mt];
+                    sum[f][mt] = zero;
+                }
+        }
+    };
+    auto read_x = [&](int buf, int u, f16x8 (&x)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const int r = 16 * mt + c, q = 4 * u + g;
+            x[mt] = *reinterpret_cast<const f16x8 *>(lds[buf] + 16 * (r * kPieces + (q ^ (r & kSwizzle))));
+        }
+    };
+
+    uint4 a0v[kLoads], a1v[kLoads];
+    f16x8 wv[2][CS][FW];
+    load_a(a0v);
+#pragma unroll
+    for (int v = 0; v < CS; v++) load_w(v, wv[0][v]);
+    load_a(a1v);
+#pragma unroll
+    for (int v = 0; v < CS; v++) load_w(v, wv[1][v]);
+    store_a(0, a0v);
+    __syncthreads();
+    // Two chunks: each computes from its buffer, with the A of the chunk after
+    // next going out first, and ends by storing the next chunk's A into the
+    // other buffer, whose readers finished before the last barrier. A step's W
+    // registers take the W of two chunks on as soon as its MFMAs have read
+    // them. The scheduling barriers keep the loads there: left alone, the
+    // compiler moves them down to just ahead of their use.
+    // step(i, v, x, w): k step v of chunk i of the pair.
+    auto pair = [&](auto step) {
+        auto chunk = [&](int i, uint4 (&a_free)[kLoads], uint4 (&a_next)[kLoads]) {
+            f16x8 x[CS][MT];
+#pragma unroll
+            for (int v = 0; v < CS; v++) read_x(i, v, x[v]);
+            load_a(a_free);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < CS; v++) {
+                step(i, v, x[v], wv[i][v]);
+                load_w(v, wv[i][v]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            store_a(i ^ 1, a_next);
+            __syncthreads();
+        };
+        chunk(0, a0v, a1v);
+        chunk(1, a1v, a0v);
+    };
+    using First = std::true_type;
+    using Later = std::false_type;
+    if constexpr (!RAGGED) {  // whole pairs of chunks per run (or pair of runs): no branch inside a pair
+        const int run_chunks = SLICES ? slice_steps / kLinearRuns / CS : steps / kLinearRuns;
+        for (int at = 0, run = 0; at < steps / CS;) {
+            pair([&](int i, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) {
+                if (i == 0 && (v == 0 || !SLICES)) mfmas(First{}, v, x, w);
+                else mfmas(Later{}, v, x, w);
+            });
+            for (at += 2; at % run_chunks != 0; at += 2)
+                pair([&](int, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) { mfmas(Later{}, v, x, w); });
+            end_runs();
+            if (SLICES && ++run == kLinearRuns) {
+                end_slice();
+                run = 0;
+            }
+        }
+    } else if constexpr (!SLICES) {
+        int b = 0;  // the chunk's first step
+        while (b < steps)
+            pair([&](int, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) {
+                if (b >= steps) return;  // the second chunk of the last pair
+                if (b + v < steps) {
+                    if (b < kLinearRuns) mfmas(First{}, v, x, w);
+                    else mfmas(Later{}, v, x, w);
+                } else if (b < kLinearRuns) {  // run b + 1 is empty
+#pragma unroll
+                    for (int f = 0; f < FW; f++)
+#pragma unroll
+                        for (int mt = 0; mt < MT; mt++) acc[kAccs - 1][f][mt] = zero;
+                }
+                if (v == 0) return;
+                if (b + kLinearRuns >= steps) end_runs();
+                b = next_chunk(b);
+            });
+    } else {
+        // Steps taken, the run in progress, its slice's first step, and the step it ends before (runs may be empty).
+        int s = 0, run = 0, slice0 = 0, run_end = 0;
+        while (run_end == 0) run_end = ++run * slice_steps / kLinearRuns;
+        bool fresh = true;  // this step starts a run
+        while (s < steps)
+            pair([&](int, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) {
+                if (s >= steps) return;
+                if (fresh) mfmas(First{}, v, x, w);
+                else mfmas(Later{}, v, x, w);
+                fresh = ++s == run_end;
+                if (!fresh) return;
+                end_runs();
+                if (s == slice0 + slice_steps) {
+                    end_slice();
+                    slice0 = s;
+                    run = 0;
+                }
+                while (run < kLinearRuns && run_end == s) run_end = slice0 + ++run * slice_steps / kLinearRuns;
+            });
+    }
+
+    // sum[f][mt][i] = C[token 16 mt + c][feature 16 (t0 + f) + 4 g + i]
+#pragma unroll
+    for (int f = 0; f < FW; f++) {
+        const int n0 = 16 * (t0 + f);
+        const bool vec_out = ((reinterpret_cast<uintptr_t>(C) & 15) | (ldc & 3)) == 0 && n0 + 16 <= N;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const f32x4 v = SLICES ? total[SLICES ? f : 0][SLICES ? mt : 0] : sum[f][mt];
+            const int tok = 16 * mt + c;
+            if (tok >= rows) continue;
+            const int64_t row = static_cast<int64_t>(m0 + tok) * ldc;
+            const int n = n0 + 4 * g;
+            if constexpr (EP == EMBER_EPILOGUE_SILU_MUL) {
+                const f16x2 h = {static_cast<f16>(clamp_half(silu(v[0]) * v[1])),
+                                 static_cast<f16>(clamp_half(silu(v[2]) * v[3]))};
+                f16 *o = static_cast<f16 *>(C) + row + n / 2;
+                if (vec_out) {
+                    *reinterpret_cast<f16x2 *>(o) = h;
+                } else {
+                    if (n + 1 < N) o[0] = h[0];
+                    if (n + 3 < N) o[1] = h[1];
+                }
+            } else if constexpr (EP == EMBER_EPILOGUE_STORE_F16) {
+                f16x4 h;
+#pragma unroll
+                for (int i = 0; i < 4; i++) h[i] = static_cast<f16>(clamp_half(v[i]));
+                f16 *o = static_cast<f16 *>(C) + row + n;
+                if (vec_out) {
+                    *reinterpret_cast<f16x4 *>(o) = h;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (n + i < N) o[i] = h[i];
+                }
+            } else {
+                constexpr bool add = EP == EMBER_EPILOGUE_ADD_F32;
+                float *o = static_cast<float *>(C) + row + n;
+                if (vec_out) {
+                    f32x4 *p = reinterpret_cast<f32x4 *>(o);
+                    *p = add ? *p + v : v;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (n + i < N) o[i] = add ? o[i] + v[i] : v[i];
+                }
+            }
+        }
+    }
+}
+
+template <int EP>
+hipError_t launch_gemm_ep(const EmberGemvArgs &a, int fw, hipStream_t stream) {
+    const int ks = a.workspace && a.workspace_bytes >= gemv_workspace_bytes(64, a.N, a.K) ? gemv_split(a.N, a.K) : 1;
+    const int slice_steps = a.K / 32 / ks;
+    const bool ragged = slice_steps % (2 * kLinearRuns * (ks > 1 ? CS : 1)) != 0;  // a run is pairs of chunks
+    const int n_blocks = (a.N + 64 * fw - 1) / (64 * fw), m_blocks = (a.M + 16 * MT - 1) / (16 * MT);
+    const f16 *A = static_cast<const f16 *>(a.A), *W = static_cast<const f16 *>(a.W);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_blocks * m_blocks)), dim3(kGemmThreads), 0, stream, A,
+                           a.lda, W, a.M, a.N, a.K, a.C, a.ldc, n_blocks, slice_steps);
+        return hipGetLastError();
+    };
+    switch ((fw == 2 ? 4 : 0) + (ks > 1 ? 2 : 0) + (ragged ? 1 : 0)) {
+        case 0: return go(gemm_kernel<1, EP, false, false>);
+        case 1: return go(gemm_kernel<1, EP, false, true>);
+        case 2: return go(gemm_kernel<1, EP, true, false>);
+        case 3: return go(gemm_kernel<1, EP, true, true>);
+        case 4: return go(gemm_kernel<2, EP, false, false>);
+        case 5: return go(gemm_kernel<2, EP, false, true>);
+        case 6: return go(gemm_kernel<2, EP, true, false>);
+        default: return go(gemm_kernel<2, EP, true, true>);
+    }
+}
+
+}  // namespace
+
+// Two feature tiles per wave read A half as often, one gives twice the
+// work-groups: two from 200 work-groups on (us, one against two: 512 x 4096 x
+// 1024, 256 work-groups of two, 10.7 / 10.5; 1800 x 1024 x 2048, 232, 18.1 /
+// 17.8; 256 x 6144 x 1024, 192, 10.4 / 10.9; 512 x 1024 x 2048, 64, 12.3 /
+// 15.4). Four spilled and were within 2% of two.
+hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
+    const int fw = (a.M + 16 * MT - 1) / (16 * MT) * ((a.N + 127) / 128) >= 200 ? 2 : 1;
+    switch (a.epilogue) {
+        case EMBER_EPILOGUE_STORE_F16: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F16>(a, fw, stream);
+        case EMBER_EPILOGUE_STORE_F32: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F32>(a, fw, stream);
+        case EMBER_EPILOGUE_ADD_F32: return launch_gemm_ep<EMBER_EPILOGUE_ADD_F32>(a, fw, stream);
+        case EMBER_EPILOGUE_SILU_MUL: return launch_gemm_ep<EMBER_EPILOGUE_SILU_MUL>(a, fw, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace ember::hip

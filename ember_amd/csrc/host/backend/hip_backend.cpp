@@ -14,8 +14,9 @@
 //     the logit rows and the LM head into f32 logits, kept on the device;
 //   - sampling and token probabilities on the device (ember_hip_sample /
 //     ember_hip_token_probs), logits copied out on request.
-// Every launch goes to one stream of default priority. Decode-sized GEMVs
-// take up to 64 rows; larger steps (prompt chunks) run them 64 rows at a time.
+// Every launch goes to one stream of default priority. The linear layers of
+// steps beyond the decode-sized GEMV's 64 rows (prompt chunks) run on the tiled
+// kernel (gemm.hip), which gives each row the GEMV's bits.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -34,6 +35,7 @@
 #include "backend/hip_paged_kv.hpp"
 #include "common/error.hpp"
 #include "ember_hip.h"
+#include "kernels.hpp"
 #include "model/safetensors.hpp"
 
 #define HIPB_CHECK(expr)                                                                            \
@@ -150,8 +152,7 @@ private:
 
 struct Linear {
     int N = 0, K = 0;
-    const void *w = nullptr;  // f16 [N, K], or packed for the GEMV (ember_hip_gemv_pack's layout)
-    bool packed = false;
+    const void *w = nullptr;  // f16 [N, K] in ember_hip_gemv_pack's layout
 };
 
 struct LayerWeights {
@@ -301,7 +302,6 @@ public:
     }
 
 private:
-    // C[M, N] (+)= A[M, K] . W^T with an epilogue, 64 rows per GEMV launch.
     // Every launch of a planned step of T tokens: embedding, the layers, then
     // the final norm and LM head of R logit rows (rows: the planned step's
     // logit rows on the device, or null for rows 0..R-1).
@@ -371,22 +371,25 @@ private:
         return true;
     }
 
+    // C[M, N] (+)= A[M, K] . W^T with an epilogue: the decode-sized kernel up to 64 rows, the tiled one beyond
+    // (the same bits per row).
     void gemm(const void *A, int lda, const Linear &W, int M, void *C, int ldc, int ep) {
-        const size_t out_elem = ep == EMBER_EPILOGUE_STORE_F32 || ep == EMBER_EPILOGUE_ADD_F32 ? 4 : 2;
-        for (int m0 = 0; m0 < M; m0 += 64) {
-            EmberGemvArgs g{};
-            g.A = static_cast<const char *>(A) + static_cast<size_t>(m0) * lda * 2;
-            g.lda = lda;
-            g.W = W.w;
-            g.M = std::min(64, M - m0);
-            g.N = W.N;
-            g.K = W.K;
-            g.C = static_cast<char *>(C) + static_cast<size_t>(m0) * ldc * out_elem;
-            g.ldc = ldc;
-            g.epilogue = ep;
-            g.workspace = gemv_ws_.get();
-            g.workspace_bytes = static_cast<int64_t>(gemv_ws_.bytes());
-            g.w_packed = W.packed ? 1 : 0;
+        EmberGemvArgs g{};
+        g.A = A;
+        g.lda = lda;
+        g.W = W.w;
+        g.M = M;
+        g.N = W.N;
+        g.K = W.K;
+        g.C = C;
+        g.ldc = ldc;
+        g.epilogue = ep;
+        g.workspace = gemv_ws_.get();
+        g.workspace_bytes = static_cast<int64_t>(gemv_ws_.bytes());
+        g.w_packed = 1;
+        if (M > 64) {
+            HIPB_CHECK(hip::launch_gemm(g, stream_));
+        } else {
             check_abi(ember_hip_gemv(&g, stream_), "gemv");
         }
     }
@@ -497,7 +500,6 @@ private:
             const std::string head = tied ? "model.embed_tokens.weight" : "lm_head.weight";
             upload_matrix(w, V, H, {{&st.get(head, {V, H}), 0, 1}}, true);
             lm_head_.w = w;
-            lm_head_.packed = true;
         }
         final_norm_ = upload_vector(st.get("model.norm.weight", {H}));
         layers_.resize(static_cast<size_t>(c.n_layers));
@@ -509,18 +511,18 @@ private:
                           {{&st.get(p + "self_attn.q_proj.weight", {Q, H}), 0, 1},
                            {&st.get(p + "self_attn.k_proj.weight", {KV, H}), Q, 1},
                            {&st.get(p + "self_attn.v_proj.weight", {KV, H}), Q + KV, 1}}, true);
-            L.qkv = {static_cast<int>(Q + 2 * KV), static_cast<int>(H), qkv, true};
+            L.qkv = {static_cast<int>(Q + 2 * KV), static_cast<int>(H), qkv};
             void *o = take(2 * prow(H) * Q);
             upload_matrix(o, H, Q, {{&st.get(p + "self_attn.o_proj.weight", {H, Q}), 0, 1}}, true);
-            L.o = {static_cast<int>(H), static_cast<int>(Q), o, true};
+            L.o = {static_cast<int>(H), static_cast<int>(Q), o};
             void *gu = take(2 * prow(2 * I) * H);
             upload_matrix(gu, 2 * I, H,
                           {{&st.get(p + "mlp.gate_proj.weight", {I, H}), 0, 2},    // even rows
                            {&st.get(p + "mlp.up_proj.weight", {I, H}), 1, 2}}, true);    // odd rows
-            L.gate_up = {static_cast<int>(2 * I), static_cast<int>(H), gu, true};
+            L.gate_up = {static_cast<int>(2 * I), static_cast<int>(H), gu};
             void *down = take(2 * prow(H) * I);
             upload_matrix(down, H, I, {{&st.get(p + "mlp.down_proj.weight", {H, I}), 0, 1}}, true);
-            L.down = {static_cast<int>(H), static_cast<int>(I), down, true};
+            L.down = {static_cast<int>(H), static_cast<int>(I), down};
             L.in_norm = upload_vector(st.get(p + "input_layernorm.weight", {H}));
             L.post_norm = upload_vector(st.get(p + "post_attention_layernorm.weight", {H}));
             if (c.qk_norm) {

@@ -27,13 +27,12 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "device.hpp"
-#include "kernels.hpp"
+#include "linear.hpp"
 
 namespace ember::hip {
 namespace {
 
-constexpr int kGemvWaves = 8;
+constexpr int kGemvWaves = kLinearRuns;  // one run of k steps per wave
 constexpr int kGemvThreads = kGemvWaves * kWave;
 constexpr int kGemvUnroll = 8;  // k steps whose W loads are in flight together, per wave
 constexpr int kGemvTargetGroups = 256;  // work-groups a launch should reach: one per CU
@@ -45,11 +44,6 @@ constexpr int kGemvSplitAbove = 4096;  // K slices at most this wide are not spl
 // with none, 6.14 with one, 5.96 with two, 6.02 with three, 6.20 with four;
 // o (one tile) 4.70, 4.65, 4.71, 4.77, 4.83.
 constexpr int gemv_early_w(int mt) { return mt == 1 ? 1 : 2; }
-// Packed W (ember_hip_gemv_pack): for each 16-feature tile and 32-wide k step,
-// the MFMA A operand as the 64 lanes take it, 8 halves per lane (lane 16 g + c:
-// row 16 tile + c, k 32 step + 8 g ..): one contiguous 1 KiB per load
-// instruction of a wave instead of 16 rows of 64 bytes. Rows past N are zero.
-constexpr int kPackBlock = 64 * 8;  // halves per (tile, k step)
 
 // Split slices are written and read with device-scope relaxed atomics (sc1
 // global stores and loads on gfx950, coherent across the XCDs' L2s), under
@@ -67,8 +61,6 @@ __device__ __forceinline__ float get_slice(const float *p) {
 __device__ __forceinline__ f16x8 load_w(const f16 *p) {
     return __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(p));  // W is read once per launch
 }
-
-__device__ __forceinline__ float silu(float g) { return g / (1.0f + expf(-g)); }
 
 // Activations staged in LDS (when the launcher passes staged): the
 // work-group's rows of A over its K slice, copied by buffer_load_dwordx4 ...
@@ -206,7 +198,8 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     // This wave's k steps (local to the slice): unsplit, w, w + 8, ...; split,
     // a contiguous run, so its consecutive loads read whole 128-byte lines of
     // a row-major W. A wave accumulates its steps in that order whatever the
-    // rounds they are issued in, so the rounds do not change the sums.
+    // rounds they are issued in, so the rounds do not change the sums
+    // (gemm_kernel keeps the same runs and the same order of their sums).
     const int steps = kw / 32;
     const int stride = SPLIT ? 1 : kGemvWaves;
     int s = SPLIT ? wave * steps / kGemvWaves : wave;
@@ -472,6 +465,8 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_wide_kernel(const f16 *__re
     }
 }
 
+}  // namespace
+
 // Work-groups per 16 features: doubled while the launch has fewer than
 // kGemvTargetGroups, the slice is wider than kGemvSplitAbove, and each slice
 // keeps at least one 32-wide k step per wave. A slice of 4096 or less runs in
@@ -489,6 +484,8 @@ int gemv_split(int N, int K) {
         ks *= 2;
     return ks;
 }
+
+namespace {
 
 // Workspace of a split launch: the merge counters (one per 16 features,
 // padded to 256 bytes), then the slice sums.

@@ -764,6 +764,48 @@ def test_gemv_packed_equals_row_major(device, M, N, KD, ep):
         assert torch.equal(outs[0].view(view), outs[1].view(view)), f"split={split}"
 
 
+def _launch_gemm(g):
+    """The library's tiled product for more than 64 rows, which HipBackend calls (no C ABI entry of its own)."""
+    import ctypes
+
+    from ember_amd import _lib
+    fn = _lib.lib()["_ZN5ember3hip11launch_gemmERK13EmberGemvArgsP12ihipStream_t"]
+    fn.argtypes, fn.restype = [ctypes.c_void_p, ctypes.c_void_p], ctypes.c_int
+    assert fn(ctypes.addressof(g), torch.cuda.current_stream().cuda_stream) == 0
+
+
+@pytest.mark.parametrize("M,N,KD", [(65, 48, 32), (127, 130, 96), (128, 4096, 1024), (200, 66, 416), (513, 1024, 3072),
+                                   (100, 2048, 6144), (70, 1040, 4352), (1801, 1024, 2048)])
+@pytest.mark.parametrize("ep", [0, 1, 2, 3])
+def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
+    """More than 64 rows on the tiled kernel: each row is the decode-sized kernel's, bit for bit, with ragged rows and
+    features, k steps that do not divide into the 8 runs (32: empty runs; 416: 13 steps), both tile widths, and the K
+    split's slices (2048 x 6144 over 2; 1040 x 4352 over 2, ragged). Features past N and rows past M stay untouched."""
+    from ember_amd import _lib
+    rng = np.random.default_rng(M + N + KD + ep)
+    a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, KD)) * 0.05).astype(np.float16)).to(device)
+    wp = K.gemv_pack(w)
+    cols = N // 2 if ep == _lib.EPILOGUE_SILU_MUL else N
+    f32 = ep in (_lib.EPILOGUE_STORE_F32, _lib.EPILOGUE_ADD_F32)
+    for ws in {None, K.gemv_workspace(64, N, KD, device)}:
+        start = torch.from_numpy(rng.standard_normal((M + 1, cols)).astype(np.float32)).to(device)
+        got = start.clone() if f32 else start.half()
+        want = got.clone()
+        g = _lib.GemvArgs()
+        g.A, g.lda, g.W, g.M, g.N, g.K = a.data_ptr(), KD, wp.data_ptr(), M, N, KD
+        g.C, g.ldc, g.epilogue, g.w_packed = got.data_ptr(), cols, ep, 1
+        if ws is not None:
+            g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
+        _launch_gemm(g)
+        for m in range(0, M, 64):
+            n = min(64, M - m)
+            K.gemv(a[m:m + n], w, want[m:m + n], ep, workspace=ws, packed=wp)
+        torch.cuda.synchronize()
+        view = torch.int32 if f32 else torch.int16
+        assert torch.equal(got.view(view), want.view(view)), f"split={ws is not None}"
+
+
 def test_gemv_saturates_f16_outputs(device):
     """store_f16 clamps to the finite f16 range instead of overflowing to inf (k_gemm.cu's to_half_sat)."""
     a = np.full((2, 64), 100.0, np.float16)
