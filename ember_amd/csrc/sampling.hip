@@ -14,12 +14,21 @@
 // so a row draws the same token in any batch). Greedy rows (temperature <=
 // 1e-5) take the first largest logit.
 //
-// Thresholds come from a radix selection over order-preserving uint32 keys of
-// v, 8 bits per pass from the top. Its histograms sum integers: counts for
-// top-k, and exp(v - max) in 2^-40 fixed point for top-p, so every bin's sum
-// is the same whatever order the LDS atomics land in, and the kept set is a
-// deterministic function of the logits (float atomics would make it depend on
-// scheduling at the boundary).
+// What bounds it: passes of one CU over the row (608 KB at 151,936 logits, 6 to
+// 10 us each), so the cuts are found in few of them. All sums are integers
+// (counts, and exp(v - max) in 2^-40 fixed point), so they are the same
+// whatever order the LDS atomics land in, and the kept set is a deterministic
+// function of the logits (float atomics would make it depend on scheduling at
+// the boundary). Three ways, the first that applies:
+//  - candidates: a lower bound of the k-th largest logit from the threads'
+//    maxima (one pass), then the few elements at or above it are collected,
+//    sorted in LDS, and every cut, the mass and the draw come from that list;
+//  - bins: a histogram over 1/64-wide steps below the maximum (one pass), then
+//    the elements of the one bin that the cut falls in are collected and sorted;
+//  - radix: 8 bits per pass over order-preserving uint32 keys of v, for bins
+//    that hold more elements than the list.
+// 16 rows of 151,936, top-k 40 and top-p 0.9: sample 27 us (303 by radix alone),
+// token_probs 25 us (276); top-p 0.95 alone, by bins: 133 us (289) and 92 (248).
 #include <cstdint>
 
 #include "device.hpp"
@@ -33,7 +42,7 @@ constexpr int kSampleWaves = kSampleThreads / kWave;
 constexpr double kFix = 1099511627776.0;  // 2^40: exp weights in (0, 1] as fixed point, V * 2^40 < 2^64
 
 __device__ __forceinline__ uint32_t order_key(float f) {  // ascending floats -> ascending keys
-    const uint32_t b = __float_as_uint(f);
+    const uint32_t b = __float_as_uint(f + 0.0f);  // -0 orders as +0
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 __device__ __forceinline__ float key_value(uint32_t k) {
@@ -54,6 +63,11 @@ __device__ __forceinline__ float gumbel_noise(uint64_t seed, uint64_t counter, u
     return -logf(-logf(u));
 }
 
+constexpr int kList = 2 * kSampleThreads;  // elements a cut's list holds
+constexpr int kBins = 2 * kSampleThreads;  // of 1 / kBinsPerUnit each, below the largest scaled logit
+constexpr float kBinsPerUnit = 64.0f;
+constexpr int kMostCandidates = 512;  // the largest top-k whose candidates are looked for
+
 struct SampleLds {
     unsigned long long hist[256];
     unsigned long long wsum[kSampleWaves];
@@ -61,6 +75,9 @@ struct SampleLds {
     int widx[kSampleWaves];
     uint32_t prefix, mask;
     unsigned long long above, at;  // after a selection: the weight above the found key, and at it
+    unsigned long long bins[kBins];
+    unsigned long long list[kList];  // elements as (key of v, ~id): descending is the order of the cuts
+    int listed;
 };
 
 // A prefix of the (v descending, id ascending) order.
@@ -114,18 +131,68 @@ __device__ unsigned long long block_sum_u64(unsigned long long v, SampleLds &sh)
     return s;
 }
 
-// First largest score(i, x[i]) over i < V (ties to the lowest index).
-template <class F>
-__device__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
-    float best = -INFINITY;
-    int idx = 0x7fffffff;
-    for_row(x, V, [&](int i, float xi) {
-        const float v = score(i, xi);
-        if (v > best) {  // i ascends per thread: the first of equal values is kept
-            best = v;
-            idx = i;
+// The sum of v over the threads before this one (and, in total, over all).
+__device__ unsigned long long block_scan_u64(unsigned long long v, SampleLds &sh, unsigned long long &total) {
+    const int lane = static_cast<int>(threadIdx.x) % kWave, wave = static_cast<int>(threadIdx.x) / kWave;
+    unsigned long long incl = v;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const unsigned long long up = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl += up;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) sh.wsum[wave] = incl;
+    __syncthreads();
+    unsigned long long before = 0;
+    total = 0;
+    for (int w = 0; w < kSampleWaves; w++) {
+        if (w < wave) before += sh.wsum[w];
+        total += sh.wsum[w];
+    }
+    return before + incl - v;
+}
+
+// The weight exp(v - mx) in (0, 1] as fixed point, rounded down: the f32
+// value's 24 significand bits, shifted (the same integer as through double).
+__device__ __forceinline__ unsigned long long fixed_weight(float v, float mx) {
+    const uint32_t b = __float_as_uint(expf(v - mx));
+    const int e = static_cast<int>(b >> 23);  // 0 (zero, subnormal) to 127; 255 for a NaN
+    const unsigned long long m = (b & 0x7fffffu) | 0x800000u;
+    const int up = e - (127 + 23 - 40);
+    return up >= 0 ? (e > 127 ? 0ull : m << up) : up > -24 && e > 0 ? m >> -up : 0ull;
+}
+
+__device__ __forceinline__ unsigned long long list_entry(float v, int i) {
+    return static_cast<unsigned long long>(order_key(v)) << 32 | static_cast<uint32_t>(~i);
+}
+__device__ __forceinline__ float entry_value(unsigned long long e) { return key_value(static_cast<uint32_t>(e >> 32)); }
+__device__ __forceinline__ int entry_id(unsigned long long e) { return static_cast<int>(~static_cast<uint32_t>(e)); }
+
+// Sorts sh.list[0, n) descending, n <= kList; every thread calls it. Entries
+// past n are overwritten with 0, which orders after every entry.
+__device__ void sort_list(int n, SampleLds &sh) {
+    const int tid = static_cast<int>(threadIdx.x);
+    int size = 2;
+    while (size < n) size *= 2;
+    __syncthreads();
+    for (int i = n + tid; i < size; i += kSampleThreads) sh.list[i] = 0;
+    __syncthreads();
+    for (int k = 2; k <= size; k *= 2)
+        for (int j = k / 2; j > 0; j /= 2) {
+            if (tid < size / 2) {  // pair (i, i + j); kList / 2 threads at most
+                const int i = 2 * tid - (tid & (j - 1));
+                const unsigned long long a = sh.list[i], b = sh.list[i + j];
+                if (((i & k) == 0) == (a < b)) {
+                    sh.list[i] = b;
+                    sh.list[i + j] = a;
+                }
+            }
+            __syncthreads();
         }
-    });
+}
+
+// The index of the threads' largest best (ties to the lowest; 0 if none is above -inf).
+__device__ int block_first_largest(float best, int idx, SampleLds &sh) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         const float ob = __shfl_xor(best, o, kWave);
@@ -152,11 +219,26 @@ __device__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
     return idx == 0x7fffffff ? 0 : idx;
 }
 
+// First largest score(i, x[i]) over i < V (ties to the lowest index).
+template <class F>
+__device__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
+    float best = -INFINITY;
+    int idx = 0x7fffffff;
+    for_row(x, V, [&](int i, float xi) {
+        const float v = score(i, xi);
+        if (v > best) {  // i ascends per thread: the first of equal values is kept
+            best = v;
+            idx = i;
+        }
+    });
+    return block_first_largest(best, idx, sh);
+}
+
 // The largest key K such that the weight of the elements with key >= K (among
 // those `within` keeps) reaches `target`; weight 1 (prob = false) or
 // exp(v - mx) in fixed point (prob = true). Returns the value of K; sh.above
 // and sh.at then hold the weight above K and at K.
-__device__ float radix_threshold(const float *x, int V, float t, const Cut &within, float mx, bool prob,
+__device__ __forceinline__ float radix_threshold(const float *x, int V, float t, const Cut within, float mx, bool prob,
                                  unsigned long long target, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
     if (tid == 0) {
@@ -173,9 +255,7 @@ __device__ float radix_threshold(const float *x, int V, float t, const Cut &with
             if (!within.keeps(v, i)) return;
             const uint32_t k = order_key(v);
             if ((k & mask) != prefix) return;
-            const unsigned long long w =
-                prob ? static_cast<unsigned long long>(static_cast<double>(expf(v - mx)) * kFix) : 1ull;
-            atomicAdd(&sh.hist[(k >> shift) & 255u], w);
+            atomicAdd(&sh.hist[(k >> shift) & 255u], prob ? fixed_weight(v, mx) : 1ull);
         });
         __syncthreads();
         if (tid < kWave) {  // wave 0 finds the digit: lane l holds bins 255 - 4l .. 252 - 4l
@@ -215,7 +295,7 @@ __device__ float radix_threshold(const float *x, int V, float t, const Cut &with
 // The r-th lowest id (r >= 1) among the elements `within` keeps whose v equals
 // theta: a radix selection over the ids, 8 bits per pass from the top, counting
 // from the lowest bin up.
-__device__ int kth_tied_id(const float *x, int V, float t, const Cut &within, float theta, unsigned long long r,
+__device__ __forceinline__ int kth_tied_id(const float *x, int V, float t, const Cut within, float theta, unsigned long long r,
                            SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
     if (tid == 0) {
@@ -266,7 +346,7 @@ __device__ int kth_tied_id(const float *x, int V, float t, const Cut &within, fl
 // The cut at the key radix_threshold just found (in sh): when the weight at
 // that key holds more tied tokens than the target still needs, only the lowest
 // ids that reach it are kept. w_each: the weight of one token at the key.
-__device__ Cut cut_at(const float *x, int V, float t, const Cut &within, float theta, unsigned long long target,
+__device__ __forceinline__ Cut cut_at(const float *x, int V, float t, const Cut within, float theta, unsigned long long target,
                       unsigned long long w_each, SampleLds &sh) {
     Cut c;
     c.theta = theta;
@@ -278,48 +358,194 @@ __device__ Cut cut_at(const float *x, int V, float t, const Cut &within, float t
     return c;
 }
 
+__device__ __forceinline__ unsigned long long top_p_target(float top_p, unsigned long long mass) {
+    const double want = ceil(static_cast<double>(top_p) * static_cast<double>(mass));
+    return want < 1.0 ? 1ull : static_cast<unsigned long long>(want);
+}
+
+// The prefix of `within` (in the cuts' order) whose weight first reaches the
+// target: `top_k` elements (top_p < 0), or top_p of the mass of `within`.
+// `kept`: the prefix's weight.
+__device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const Cut within, float mx, int top_k,
+                                          float top_p, unsigned long long &kept, SampleLds &sh) {
+    const int tid = static_cast<int>(threadIdx.x);
+    const bool prob = top_p >= 0.0f;
+    // (mx - v) rounds the same way for equal v and never orders two v the other way round, so bins follow the order
+    // (with an infinite mx, every element is in the last one).
+    auto bin_of = [&](float v) {
+        const float d = (mx - v) * kBinsPerUnit;
+        return d < static_cast<float>(kBins - 1) ? static_cast<int>(d) : kBins - 1;
+    };
+    __syncthreads();
+    for (int i = tid; i < kBins; i += kSampleThreads) sh.bins[i] = 0;
+    if (tid == 0) sh.listed = 0;
+    __syncthreads();
+    for_row(x, V, [&](int i, float xi) {
+        const float v = xi / t;
+        if (!within.keeps(v, i)) return;
+        const unsigned long long w = prob ? fixed_weight(v, mx) : 1ull;
+        if (w) atomicAdd(&sh.bins[bin_of(v)], w);
+    });
+    __syncthreads();
+    const unsigned long long b0 = sh.bins[2 * tid], b1 = sh.bins[2 * tid + 1];
+    unsigned long long total;
+    const unsigned long long before = block_scan_u64(b0 + b1, sh, total);
+    const unsigned long long target = prob ? top_p_target(top_p, total) : static_cast<unsigned long long>(top_k);
+    if (before < target && before + b0 + b1 >= target) {  // one thread (none if the total falls short)
+        sh.prefix = static_cast<uint32_t>(2 * tid + (before + b0 >= target ? 0 : 1));
+        sh.above = before + (before + b0 >= target ? 0 : b0);
+    }
+    __syncthreads();
+    kept = total;
+    const bool none = prob && total == 0;  // an infinite maximum: nothing has weight, which the radix search settles
+    if (total < target && !none) return within;
+    const int bin = none ? kBins : static_cast<int>(sh.prefix);
+    const unsigned long long above = sh.above;
+    for_row(x, V, [&](int i, float xi) {
+        const float v = xi / t;
+        if (!within.keeps(v, i) || bin_of(v) != bin) return;
+        const int at = atomicAdd(&sh.listed, 1);
+        if (at < kList) sh.list[at] = list_entry(v, i);
+    });
+    __syncthreads();
+    const int n = sh.listed;
+    Cut c;
+    if (n <= kList && !none) {
+        sort_list(n, sh);
+        const unsigned long long e0 = 2 * tid < n ? sh.list[2 * tid] : 0, e1 = 2 * tid + 1 < n ? sh.list[2 * tid + 1] : 0;
+        const unsigned long long w0 = 2 * tid < n ? (prob ? fixed_weight(entry_value(e0), mx) : 1ull) : 0;
+        const unsigned long long w1 = 2 * tid + 1 < n ? (prob ? fixed_weight(entry_value(e1), mx) : 1ull) : 0;
+        unsigned long long all;
+        const unsigned long long pre = above + block_scan_u64(w0 + w1, sh, all);
+        __syncthreads();
+        if (pre < target && pre + w0 + w1 >= target) {
+            const bool first = pre + w0 >= target;
+            sh.list[0] = first ? e0 : e1;  // every thread has read its entries
+            sh.above = pre + (first ? w0 : w0 + w1);
+        }
+        __syncthreads();
+        c.theta = entry_value(sh.list[0]);
+        c.id_cut = entry_id(sh.list[0]);
+        kept = sh.above;
+        return c;
+    }
+    const float theta = radix_threshold(x, V, t, within, mx, prob, target, sh);
+    const unsigned long long w_each = prob ? fixed_weight(theta, mx) : 1ull, over = sh.above, at = sh.at;
+    const unsigned long long need = w_each == 0 || target <= over ? 0 : (target - over + w_each - 1) / w_each;
+    kept = over + (need && need * w_each < at ? need * w_each : at);
+    return cut_at(x, V, t, within, theta, target, w_each, sh);
+}
+
 struct Dist {
     bool greedy;
     float t, mx, min_w;
     Cut k, p;              // the top-k and top-p cuts (the top-p one lies inside the top-k one)
-    unsigned long long z;  // fixed-point mass of the kept set
+    unsigned long long z;  // fixed-point mass of the kept set (where asked for)
+    int listed;            // the kept set is within sh.list[0, listed), sorted; 0: not listed
     __device__ bool keeps(float v, int i) const { return k.keeps(v, i) && p.keeps(v, i) && expf(v - mx) >= min_w; }
 };
 
-__device__ __forceinline__ unsigned long long fixed_weight(float v, float mx) {
-    return static_cast<unsigned long long>(static_cast<double>(expf(v - mx)) * kFix);
+// Rows whose kept set is among few elements: those at or above a bound that
+// the threads' maxima give. top-k: at least top_k threads (ceil(top_k / 16) of
+// each wave's) have a maximum at or above it, so the top_k first elements do.
+// Otherwise min-p: nothing below max + ln(min_p) is kept. Returns false, with
+// nothing settled, when the bound lets too many through.
+__device__ __forceinline__ bool few_candidates(const float *x, int V, const EmberSampleParams &p, float thread_max, Dist &d,
+                               SampleLds &sh) {
+    const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave, wave = tid / kWave;
+    const bool by_k = p.top_k > 0 && p.top_k <= kMostCandidates && p.top_k < V;
+    const bool by_min_p = !by_k && (p.top_k <= 0 || p.top_k >= V) && !(p.top_p < 1.0f) && d.min_w > 0.0f && d.min_w <= 1.0f;
+    if (!by_k && !by_min_p) return false;
+    float bound;
+    if (by_k) {
+        float m = thread_max;  // the wave's maxima, sorted descending over its lanes
+        for (int k = 2; k <= kWave; k *= 2)
+            for (int j = k / 2; j > 0; j /= 2) {
+                const float o = __shfl_xor(m, j, kWave);
+                const bool larger = ((lane & j) == 0) == ((lane & k) == 0);  // this lane keeps the larger of the two
+                m = larger ? fmaxf(m, o) : fminf(m, o);
+            }
+        const float mine = __shfl(m, (p.top_k + kSampleWaves - 1) / kSampleWaves - 1, kWave);
+        bound = -block_max(-mine, sh);
+        // Quotients of nearby logits can be equal: elements within rounding of the bound count too.
+        bound -= fabsf(bound) * 0x1p-20f + 1e-30f;
+    } else {
+        bound = (d.mx + logf(d.min_w) - 0.01f - fabsf(d.mx) * 0x1p-20f) * d.t;  // well below the cut
+    }
+    if (!(bound / d.t > -INFINITY)) return false;  // quotients that overflow are all equal
+    __syncthreads();
+    if (tid == 0) sh.listed = 0;
+    __syncthreads();
+    for_row(x, V, [&](int i, float xi) {
+        if (!(xi >= bound)) return;
+        const int at = atomicAdd(&sh.listed, 1);
+        if (at < kList) sh.list[at] = list_entry(xi / d.t, i);
+    });
+    __syncthreads();
+    const int n = sh.listed;
+    if (n > kList || n == 0) return false;
+    sort_list(n, sh);
+    const int kk = by_k ? min(p.top_k, n) : n;  // the top-k set: list[0, kk)
+    // Each thread's two entries, their weights, and the mass before them.
+    const int i0 = 2 * tid, i1 = 2 * tid + 1;
+    const float v0 = i0 < kk ? entry_value(sh.list[i0]) : 0.0f, v1 = i1 < kk ? entry_value(sh.list[i1]) : 0.0f;
+    const unsigned long long w0 = i0 < kk ? fixed_weight(v0, d.mx) : 0, w1 = i1 < kk ? fixed_weight(v1, d.mx) : 0;
+    unsigned long long zk;
+    const unsigned long long before = block_scan_u64(w0 + w1, sh, zk);
+    int keep = kk;  // the top-p set: list[0, keep)
+    if (p.top_p < 1.0f) {
+        const unsigned long long target = top_p_target(p.top_p, zk);
+        __syncthreads();
+        if (before < target && before + w0 + w1 >= target)  // one thread
+            sh.prefix = static_cast<uint32_t>(before + w0 >= target ? i0 + 1 : i1 + 1);
+        __syncthreads();
+        keep = static_cast<int>(sh.prefix);
+    }
+    if (by_k) {
+        d.k.theta = entry_value(sh.list[kk - 1]);
+        d.k.id_cut = entry_id(sh.list[kk - 1]);
+    }
+    if (p.top_p < 1.0f) {
+        d.p.theta = entry_value(sh.list[keep - 1]);
+        d.p.id_cut = entry_id(sh.list[keep - 1]);
+    }
+    d.listed = keep;
+    d.z = block_sum_u64((i0 < keep && expf(v0 - d.mx) >= d.min_w ? w0 : 0) + (i1 < keep && expf(v1 - d.mx) >= d.min_w ? w1 : 0), sh);
+    return true;
 }
 
-// The kept set of one row, in the host sampler's order.
-__device__ Dist distribution(const float *x, int V, const EmberSampleParams &p, SampleLds &sh) {
+// The kept set of one row, in the host sampler's order; its mass if `mass`.
+__device__ __forceinline__ Dist distribution(const float *x, int V, const EmberSampleParams &p, bool mass, SampleLds &sh) {
     Dist d{};
     d.greedy = !(p.temperature > 1e-5f);
     if (d.greedy) return d;
     d.t = p.temperature;
     float m = -INFINITY;
-    for_row(x, V, [&](int, float xi) { m = fmaxf(m, xi / d.t); });
-    d.mx = block_max(m, sh);
+    for_row(x, V, [&](int, float xi) { m = fmaxf(m, xi); });
+    d.mx = block_max(m, sh) / d.t;  // the largest quotient: division by t > 0 keeps the order
+    d.min_w = p.min_p > 0.0f ? p.min_p : 0.0f;
     const Cut all;
     d.k = all;
     d.p = all;
-    if (p.top_k > 0 && p.top_k < V) {
-        const auto target = static_cast<unsigned long long>(p.top_k);
-        const float theta = radix_threshold(x, V, d.t, all, d.mx, false, target, sh);
-        d.k = cut_at(x, V, d.t, all, theta, target, 1ull, sh);
+    if (fabsf(d.mx) < INFINITY && d.t < 1e5f && few_candidates(x, V, p, m, d, sh)) return d;
+    unsigned long long kept = 0;  // weight of the set so far
+    bool known = false;           // and it is the kept set's mass
+#pragma unroll 1
+    for (int which = 0; which < 2; which++) {
+        if (which == 0 ? !(p.top_k > 0 && p.top_k < V) : !(p.top_p < 1.0f)) continue;
+        const Cut c = prefix_cut(x, V, d.t, which == 0 ? all : d.k, d.mx, p.top_k, which == 0 ? -1.0f : fmaxf(p.top_p, 0.0f),
+                                 kept, sh);
+        if (which == 0) {
+            d.k = c;
+        } else {
+            d.p = c;
+            known = d.min_w == 0.0f;
+        }
     }
-    if (p.top_p < 1.0f) {
-        unsigned long long s = 0;
-        for_row(x, V, [&](int i, float xi) {
-            const float v = xi / d.t;
-            if (d.k.keeps(v, i)) s += fixed_weight(v, d.mx);
-        });
-        const unsigned long long zk = block_sum_u64(s, sh);
-        const double want = ceil(static_cast<double>(p.top_p) * static_cast<double>(zk));
-        const unsigned long long target = want < 1.0 ? 1ull : static_cast<unsigned long long>(want);
-        const float theta = radix_threshold(x, V, d.t, d.k, d.mx, true, target, sh);
-        d.p = cut_at(x, V, d.t, d.k, theta, target, fixed_weight(theta, d.mx), sh);
+    if (known || !mass) {
+        d.z = kept;
+        return d;
     }
-    d.min_w = p.min_p > 0.0f ? p.min_p : 0.0f;
     // the kept set's mass (min-p applied), for token probabilities
     unsigned long long s = 0;
     for_row(x, V, [&](int i, float xi) {
@@ -337,10 +563,23 @@ __global__ void __launch_bounds__(kSampleThreads) sample_kernel(const float *__r
     const int r = static_cast<int>(blockIdx.x);
     const float *x = logits + static_cast<int64_t>(r) * V;
     const EmberSampleParams p = params[r];
-    const Dist d = distribution(x, V, p, sh);
+    const Dist d = distribution(x, V, p, false, sh);
     int tok;
     if (d.greedy) {
         tok = block_argmax(x, V, [](int, float xi) { return xi; }, sh);
+    } else if (d.listed) {
+        float best = -INFINITY;
+        int idx = 0x7fffffff;
+        for (int j = static_cast<int>(threadIdx.x); j < d.listed; j += kSampleThreads) {
+            const float v = entry_value(sh.list[j]);
+            const int i = entry_id(sh.list[j]);
+            const float s = expf(v - d.mx) >= d.min_w ? v + gumbel_noise(p.seed, p.counter, static_cast<uint32_t>(i)) : -INFINITY;
+            if (s > best || (s == best && s > -INFINITY && i < idx)) {
+                best = s;
+                idx = i;
+            }
+        }
+        tok = block_first_largest(best, idx, sh);
     } else {
         tok = block_argmax(x, V, [&](int i, float xi) {
             const float v = xi / d.t;
@@ -363,7 +602,7 @@ __global__ void __launch_bounds__(kSampleThreads) prob_kernel(const float *__res
     }
     const float *x = logits + static_cast<int64_t>(r) * V;
     const EmberSampleParams p = params[r];
-    const Dist d = distribution(x, V, p, sh);
+    const Dist d = distribution(x, V, p, true, sh);
     float prob;
     if (d.greedy) {
         prob = block_argmax(x, V, [](int, float xi) { return xi; }, sh) == tok ? 1.0f : 0.0f;

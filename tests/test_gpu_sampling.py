@@ -146,3 +146,55 @@ def test_ties_at_the_top_k_and_top_p_cuts(case):
     toks = gpu_sample(np.tile(x, (R, 1)), [(t, top_p, top_k, min_p, 31, c) for c in range(R)])
     assert set(toks) <= set(kept.tolist()), "a draw outside the host's kept set"
     assert toks[:100] == [oracle.sample(x, t, top_p, top_k, min_p, seed=31, counter=c) for c in range(100)]
+
+
+def _row(kind, V, rng):
+    if kind == "flat":
+        return rng.normal(0.0, 2.0, V).astype(np.float32)
+    if kind == "peaked":  # a few dozen likely tokens well above a broad floor
+        x = rng.normal(0.0, 2.0, V).astype(np.float32)
+        x[rng.integers(0, V, 40)] += rng.uniform(6.0, 14.0, 40).astype(np.float32)
+        return x
+    if kind == "tied":  # steps of 1/8: thousands of equal logits, -0 and +0 among them
+        return (np.round(rng.normal(0.0, 1.0, V) * 8) / 8).astype(np.float32)
+    x = np.full(V, -np.inf, np.float32)  # "masked": 30 tokens allowed
+    x[rng.choice(V, 30, replace=False)] = rng.normal(0.0, 2.0, 30).astype(np.float32)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["flat", "peaked", "tied", "masked"])
+@pytest.mark.parametrize("V", [40, 1023, 4999, 151936])
+def test_every_way_to_the_cuts_keeps_the_hosts_set(kind, V):
+    """Top-k from the threads' maxima (k 1 to 512), through bins (beyond) and by radix (bins with more ties than the
+    list), top-p alone and inside top-k, min-p alone and after them: the draws are the host sampler's, and the tokens
+    either side of the cut have the host's probabilities (the first left out: 0)."""
+    rng = np.random.default_rng(V + len(kind))
+    x = _row(kind, V, rng)
+    forms = [(0.8, 0.9, 40, 0.0), (1.0, 1.0, 1, 0.0), (0.6, 0.95, 20, 0.05), (0.9, 1.0, 512, 0.0), (0.9, 0.7, 513, 0.0),
+             (1.1, 1.0, 3000, 0.01), (1.0, 0.95, 0, 0.0), (0.7, 0.5, 0, 0.02), (1.2, 1.0, 0, 0.02), (1e-3, 0.9, 40, 0.0)]
+    rows, queries, want = [], [], []
+    for i, (t, top_p, top_k, min_p) in enumerate(forms):
+        kept, probs = oracle.sampling_distribution(x, t, top_p, top_k, min_p)
+        rows.append((t, top_p, top_k, min_p, 77, 0))
+        left = np.setdiff1d(np.argsort(-x, kind="stable")[:len(kept) + 4], kept)
+        for tok, p in [*zip(kept[:3], probs[:3]), *zip(kept[-3:], probs[-3:]), *((tok, 0.0) for tok in left[:4])]:
+            queries.append((i, int(tok)))
+            want.append(p)
+    got = gpu_probs(np.tile(x, (len(forms), 1)), rows, queries)
+    np.testing.assert_allclose(got, np.array(want, np.float32), rtol=2e-4, atol=1e-9)
+    draws = [r[:5] + (c,) for r in rows for c in range(4)]
+    toks = gpu_sample(np.tile(x, (len(draws), 1)), draws)
+    assert toks == [oracle.sample(x, *r[:4], seed=r[4], counter=r[5]) for r in draws]
+
+
+def test_rows_with_infinities_and_nan():
+    """A NaN logit is never drawn, as if it were -inf."""
+    rng = np.random.default_rng(3)
+    x = rng.normal(0.0, 2.0, 5000).astype(np.float32)
+    clean = x.copy()
+    x[[0, 17, 4999]] = np.nan
+    clean[[0, 17, 4999]] = -np.inf
+    forms = [(0.8, 0.9, 40, 0.0, 9, 1), (1.0, 0.9, 0, 0.0, 9, 2), (1.0, 1.0, 900, 0.0, 9, 3), (1.2, 1.0, 0, 0.02, 9, 4)]
+    assert gpu_sample(np.tile(x, (4, 1)), forms) == gpu_sample(np.tile(clean, (4, 1)), forms)
+    everything = np.full(5000, -np.inf, np.float32)  # nothing to choose from: token 0, as for a greedy row of NaN
+    assert gpu_sample(np.tile(everything, (4, 1)), forms) == [0] * 4
