@@ -1,6 +1,7 @@
 // The linear layers of a prompt on gfx950: C[M, N] = A[M, K] . W[N, K]^T for
-// more rows than the decode-sized kernel takes (linear.hip, 64), with the same
-// four epilogues and the same bits per row (linear.hpp: the order of the sums).
+// more rows than the decode-sized kernel takes (linear.hip, 64), and for wide
+// batches of up to 64 where it is the faster one, with the same four epilogues
+// and the same bits per row (linear.hpp: the order of the sums).
 //
 // What bounds it: the matrix cores, once W and A are re-read little enough; at
 // few tokens, one work-group's chain of chunks. A work-group of 4 waves covers
@@ -14,9 +15,9 @@
 //
 // Measured (packed W, a graph of 60 launches over 8 weights), against 64 rows
 // per launch of the decode-sized kernel: 1800 x 4096 x 1024 26.4 us (572
-// TFLOP/s), 129 before; 1800 x 1024 x 2048 17.8, 122; 1800 x 6144 x 1024 40.3,
-// 233; 1800 x 1024 x 3072 23.1, 166; 256 x 4096 x 1024 8.3, 19.8; 256 x 1024 x
-// 2048 11.9, 17.2. A 1800-token prompt of the 28-layer model: 19.93 -> 4.86 ms.
+// TFLOP/s), 129 before; 1800 x 1024 x 2048 17.9, 121; 1800 x 6144 x 1024 40.8,
+// 229; 1800 x 1024 x 3072 22.9, 163; 256 x 4096 x 1024 7.7, 19.1; 256 x 1024 x
+// 2048 9.4, 16.8; 48 x 12288 x 2048 15.4, 27.3; 64 x 151936 x 1024 72, 135.
 #include <algorithm>
 #include <type_traits>
 
@@ -25,26 +26,73 @@
 namespace ember::hip {
 namespace {
 
-constexpr int kGemmWaves = 4;
-constexpr int kGemmThreads = kGemmWaves * kWave;
-constexpr int MT = 4;  // 16-token tiles per work-group
-constexpr int CS = 2;  // k steps per LDS chunk of A
+constexpr int kGemmWaves = 4;                      // of one K group: side by side over the features
+constexpr int kGemmThreads = kGemmWaves * kWave;  // of one K group
+constexpr int CS = 2;                             // k steps per LDS chunk of A
+constexpr int kSplitGroups = 4;                   // K groups of the split form
 constexpr int kXcds = 8;
 constexpr int kDescWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
 
-// SLICES: K is split in KS slices as the decode-sized kernel splits this shape.
-template <int FW, int EP, bool SLICES, bool RAGGED>
-__global__ void __launch_bounds__(kGemmThreads, 2)
-    gemm_kernel(const f16 *__restrict__ A, int lda, const f16 *__restrict__ W, int M, int N, int K,
-                void *__restrict__ C, int ldc, int n_blocks, int slice_steps) {
+// One lane's four adjacent outputs (features n .. n + 3 of one token; all below N if vec_out).
+template <int EP>
+__device__ __forceinline__ void store_outputs(void *C, int64_t row, int n, int N, const f32x4 v, bool vec_out) {
+    if constexpr (EP == EMBER_EPILOGUE_SILU_MUL) {
+        const f16x2 h = {static_cast<f16>(clamp_half(silu(v[0]) * v[1])), static_cast<f16>(clamp_half(silu(v[2]) * v[3]))};
+        f16 *o = static_cast<f16 *>(C) + row + n / 2;
+        if (vec_out) {
+            *reinterpret_cast<f16x2 *>(o) = h;
+        } else {
+            if (n + 1 < N) o[0] = h[0];
+            if (n + 3 < N) o[1] = h[1];
+        }
+    } else if constexpr (EP == EMBER_EPILOGUE_STORE_F16) {
+        f16x4 h;
+#pragma unroll
+        for (int i = 0; i < 4; i++) h[i] = static_cast<f16>(clamp_half(v[i]));
+        f16 *o = static_cast<f16 *>(C) + row + n;
+        if (vec_out) {
+            *reinterpret_cast<f16x4 *>(o) = h;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (n + i < N) o[i] = h[i];
+        }
+    } else {
+        constexpr bool add = EP == EMBER_EPILOGUE_ADD_F32;
+        float *o = static_cast<float *>(C) + row + n;
+        if (vec_out) {
+            f32x4 *p = reinterpret_cast<f32x4 *>(o);
+            *p = add ? *p + v : v;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (n + i < N) o[i] = add ? o[i] + v[i] : v[i];
+        }
+    }
+}
+
+// MT tiles of 16 tokens and 4 x FW of 16 features per work-group. KG = 1: four
+// waves take all of K; SLICES: K is in slices as the decode-sized kernel splits
+// this shape. KG = 4: four K groups of four waves, group k summing runs 2 k and
+// 2 k + 1 side by side; the runs' sums meet in LDS and are added in run order.
+// RAGGED: the runs are not whole pairs of chunks.
+template <int MT, int FW, int KG, int EP, bool SLICES, bool RAGGED>
+__global__ void __launch_bounds__(kGemmThreads *KG, KG == 1 ? 2 : 1)
+    gemm_kernel(const f16 *__restrict__ A, int lda, const f16 *__restrict__ W, int w_step, int64_t w_tile, int M, int N,
+                int K, void *__restrict__ C, int ldc, int n_blocks, int slice_steps) {
+    static_assert(KG == 1 || (KG == kSplitGroups && FW == 1 && !SLICES));
     constexpr int kRows = 16 * MT;
     constexpr int kPieces = CS * 4;  // 16-byte pieces of a row per chunk of CS k steps
     constexpr int kSwizzle = kPieces < 16 ? kPieces - 1 : 15;
     constexpr int kLoads = kRows * kPieces / kGemmThreads;  // 16-byte pieces of A per thread and chunk
     static_assert(kRows * kPieces % kGemmThreads == 0 && (CS & (CS - 1)) == 0);
-    __shared__ __align__(16) unsigned char lds[2][kRows * kPieces * 16];
-    const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave;
+    constexpr int kBufBytes = kRows * kPieces * 16;
+    constexpr int kSumBytes = KG == 1 ? 0 : kLinearRuns * kGemmWaves * MT * kWave * 16;  // the runs' sums
+    __shared__ __align__(16) unsigned char lds_all[kSumBytes > 2 * KG * kBufBytes ? kSumBytes : 2 * KG * kBufBytes];
+    const int tid = static_cast<int>(threadIdx.x) % kGemmThreads, lane = tid % kWave;  // in the K group
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kGemmThreads);
+    auto lds = [&](int buf) { return lds_all + (kg * 2 + buf) * kBufBytes; };
     const int c = lane % 16, g = lane / 16;
     // Block id -> (token block, feature block). Ids that differ by a multiple
     // of 8 run on one XCD: with feature blocks in multiples of 8, an XCD takes
@@ -76,22 +124,25 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
         aoff[j] = r < rows ? static_cast<uint32_t>(r * lda + 8 * q) * 2u : records;
         aslot[j] = 16 * (r * kPieces + (q ^ (r & kSwizzle)));
     }
+    // W: packed, a tile's k steps are 1 KiB blocks in lane order; row-major, this lane's row (rows past N repeat the last).
     const f16 *w[FW];
 #pragma unroll
     for (int f = 0; f < FW; f++)
-        w[f] = W + static_cast<int64_t>(min(t0 + f, tiles - 1)) * steps * kPackBlock + 8 * lane;
+        w[f] = w_tile ? W + min(t0 + f, tiles - 1) * w_tile + 8 * lane
+                      : W + static_cast<int64_t>(min(16 * (t0 + f) + c, N - 1)) * K + 8 * g;
 
     // A chunk is two adjacent k steps (128 bytes of a row of A). Unsplit, they
     // belong to runs 2 p and 2 p + 1, which are summed side by side: chunks 2 p,
     // 2 p + 8, ..., then the next pair of runs. In a slice they follow each
-    // other in one run. next_chunk(b): the chunk after the one at step b (S: none).
+    // other in one run. A K group takes one pair of runs. next_chunk(b): the chunk after the one at step b (S: none).
     auto next_chunk = [&](int b) {
         if (SLICES) return b + 2;
+        if (KG > 1) return min(b + kLinearRuns, steps);
         return b + kLinearRuns < steps ? b + kLinearRuns
                : b < steps && b % kLinearRuns + 2 < min(kLinearRuns, steps) ? b % kLinearRuns + 2
                                                                             : steps;
     };
-    int a_chunk = 0;  // the chunk that load_a takes next
+    int a_chunk = min(2 * kg, steps);  // the chunk that load_a takes next
     auto load_a = [&](uint4 (&v)[kLoads]) {
         const uint32_t k = 64u * static_cast<uint32_t>(a_chunk);
         a_chunk = next_chunk(a_chunk);
@@ -101,11 +152,11 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
     };
     auto store_a = [&](int buf, const uint4 (&v)[kLoads]) {
 #pragma unroll
-        for (int j = 0; j < kLoads; j++) *reinterpret_cast<uint4 *>(lds[buf] + aslot[j]) = v[j];
+        for (int j = 0; j < kLoads; j++) *reinterpret_cast<uint4 *>(lds(buf) + aslot[j]) = v[j];
     };
-    int w_chunk = 0;  // the chunk whose W goes out next
+    int w_chunk = min(2 * kg, steps);  // the chunk whose W goes out next
     auto load_w = [&](int v, f16x8 (&wv)[FW]) {
-        const int64_t at = static_cast<int64_t>(min(w_chunk + v, steps - 1)) * kPackBlock;
+        const int64_t at = static_cast<int64_t>(min(w_chunk + v, steps - 1)) * w_step;
         if (v == CS - 1) w_chunk = next_chunk(w_chunk);
 #pragma unroll
         for (int f = 0; f < FW; f++) wv[f] = *reinterpret_cast<const f16x8 *>(w[f] + at);
@@ -113,14 +164,14 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
 
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     constexpr int kAccs = SLICES ? 1 : 2;  // runs summed side by side
-    f32x4 acc[kAccs][FW][MT], sum[FW][MT], total[SLICES ? FW : 1][SLICES ? MT : 1];
+    f32x4 acc[kAccs][FW][MT], sum[KG == 1 ? FW : 1][KG == 1 ? MT : 1], total[SLICES ? FW : 1][SLICES ? MT : 1];
 #pragma unroll
     for (int f = 0; f < FW; f++)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
 #pragma unroll
             for (int r = 0; r < kAccs; r++) acc[r][f][mt] = zero;
-            sum[f][mt] = zero;
+            if constexpr (KG == 1) sum[f][mt] = zero;
             if constexpr (SLICES) total[f][mt] = zero;
         }
     // The MFMAs of a chunk's k step v: every tile of the wave, from zero at the start of a run.
@@ -134,12 +185,14 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
                                                                    0, 0, 0);
     };
     auto end_runs = [&]() {  // the runs' sums join the slice's
+        if constexpr (KG == 1) {
 #pragma unroll
         for (int r = 0; r < kAccs; r++)
 #pragma unroll
             for (int f = 0; f < FW; f++)
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) sum[f][mt] = sum[f][mt] + acc[r][f][mt];
+        }
     };
     auto end_slice = [&]() {  // the slice's sum joins the total
         if constexpr (SLICES) {
@@ -156,7 +209,7 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
             const int r = 16 * mt + c, q = 4 * u + g;
-            x[mt] = *reinterpret_cast<const f16x8 *>(lds[buf] + 16 * (r * kPieces + (q ^ (r & kSwizzle))));
+            x[mt] = *reinterpret_cast<const f16x8 *>(lds(buf) + 16 * (r * kPieces + (q ^ (r & kSwizzle))));
         }
     };
 
@@ -198,7 +251,13 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
     };
     using First = std::true_type;
     using Later = std::false_type;
-    if constexpr (!RAGGED) {  // whole pairs of chunks per run (or pair of runs): no branch inside a pair
+    if constexpr (KG > 1) {  // one pair of runs, from zero; the groups take the same number of pairs
+        for (int b = 2 * kg, at = 0; at < steps; at += 2 * kLinearRuns)
+            pair([&](int, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) {
+                if (!RAGGED || b + v < steps) mfmas(Later{}, v, x, w);
+                if (RAGGED && v == CS - 1) b += kLinearRuns;
+            });
+    } else if constexpr (!RAGGED) {  // whole pairs of chunks per run (or pair of runs): no branch inside a pair
         const int run_chunks = SLICES ? slice_steps / kLinearRuns / CS : steps / kLinearRuns;
         for (int at = 0, run = 0; at < steps / CS;) {
             pair([&](int i, int v, const f16x8 (&x)[MT], const f16x8 (&w)[FW]) {
@@ -254,93 +313,99 @@ __global__ void __launch_bounds__(kGemmThreads, 2)
     }
 
     // sum[f][mt][i] = C[token 16 mt + c][feature 16 (t0 + f) + 4 g + i]
+    const auto whole = [&](int n0) { return ((reinterpret_cast<uintptr_t>(C) & 15) | (ldc & 3)) == 0 && n0 + 16 <= N; };
+    if constexpr (KG > 1) {
+        // Every group is past the last chunk's barrier: the buffers take the runs' sums, and group k adds and stores
+        // token tile k.
+        f32x4 *sums = reinterpret_cast<f32x4 *>(lds_all) + wave * MT * kWave + lane;  // [run][wave][mt][lane]
+        constexpr int kRunSums = kGemmWaves * MT * kWave;
 #pragma unroll
-    for (int f = 0; f < FW; f++) {
-        const int n0 = 16 * (t0 + f);
-        const bool vec_out = ((reinterpret_cast<uintptr_t>(C) & 15) | (ldc & 3)) == 0 && n0 + 16 <= N;
+        for (int r = 0; r < kAccs; r++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const f32x4 v = SLICES ? total[SLICES ? f : 0][SLICES ? mt : 0] : sum[f][mt];
-            const int tok = 16 * mt + c;
-            if (tok >= rows) continue;
-            const int64_t row = static_cast<int64_t>(m0 + tok) * ldc;
-            const int n = n0 + 4 * g;
-            if constexpr (EP == EMBER_EPILOGUE_SILU_MUL) {
-                const f16x2 h = {static_cast<f16>(clamp_half(silu(v[0]) * v[1])),
-                                 static_cast<f16>(clamp_half(silu(v[2]) * v[3]))};
-                f16 *o = static_cast<f16 *>(C) + row + n / 2;
-                if (vec_out) {
-                    *reinterpret_cast<f16x2 *>(o) = h;
-                } else {
-                    if (n + 1 < N) o[0] = h[0];
-                    if (n + 3 < N) o[1] = h[1];
-                }
-            } else if constexpr (EP == EMBER_EPILOGUE_STORE_F16) {
-                f16x4 h;
+            for (int mt = 0; mt < MT; mt++) sums[(2 * kg + r) * kRunSums + mt * kWave] = acc[r][0][mt];
+        __syncthreads();
+        const int tok = 16 * kg + c;
+        if (kg >= MT || tok >= rows) return;
+        f32x4 v = zero;
 #pragma unroll
-                for (int i = 0; i < 4; i++) h[i] = static_cast<f16>(clamp_half(v[i]));
-                f16 *o = static_cast<f16 *>(C) + row + n;
-                if (vec_out) {
-                    *reinterpret_cast<f16x4 *>(o) = h;
-                } else {
+        for (int r = 0; r < kLinearRuns; r++) v = v + sums[r * kRunSums + kg * kWave];
+        store_outputs<EP>(C, static_cast<int64_t>(m0 + tok) * ldc, 16 * t0 + 4 * g, N, v, whole(16 * t0));
+    } else {
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (n + i < N) o[i] = h[i];
-                }
-            } else {
-                constexpr bool add = EP == EMBER_EPILOGUE_ADD_F32;
-                float *o = static_cast<float *>(C) + row + n;
-                if (vec_out) {
-                    f32x4 *p = reinterpret_cast<f32x4 *>(o);
-                    *p = add ? *p + v : v;
-                } else {
+        for (int f = 0; f < FW; f++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (n + i < N) o[i] = add ? o[i] + v[i] : v[i];
-                }
+            for (int mt = 0; mt < MT; mt++) {
+                const int tok = 16 * mt + c;
+                if (tok >= rows) continue;
+                store_outputs<EP>(C, static_cast<int64_t>(m0 + tok) * ldc, 16 * (t0 + f) + 4 * g, N,
+                                  SLICES ? total[SLICES ? f : 0][SLICES ? mt : 0] : sum[f][mt], whole(16 * (t0 + f)));
             }
-        }
     }
 }
 
+// form: 0 the split form, 1 or 2 feature tiles per wave of the other.
 template <int EP>
-hipError_t launch_gemm_ep(const EmberGemvArgs &a, int fw, hipStream_t stream) {
-    const int ks = a.workspace && a.workspace_bytes >= gemv_workspace_bytes(64, a.N, a.K) ? gemv_split(a.N, a.K) : 1;
-    const int slice_steps = a.K / 32 / ks;
+hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, hipStream_t stream) {
+    const int ks = form > 0 && a.workspace ? gemv_split(a.N, a.K) : 1;
+    const int steps = a.K / 32, slice_steps = steps / ks;
     const bool ragged = slice_steps % (2 * kLinearRuns * (ks > 1 ? CS : 1)) != 0;  // a run is pairs of chunks
-    const int n_blocks = (a.N + 64 * fw - 1) / (64 * fw), m_blocks = (a.M + 16 * MT - 1) / (16 * MT);
+    const int mt = form > 0 || a.M > 32 ? 4 : 2;
+    const int fw = std::max(form, 1);
+    const int n_blocks = (a.N + 64 * fw - 1) / (64 * fw), m_blocks = (a.M + 16 * mt - 1) / (16 * mt);
     const f16 *A = static_cast<const f16 *>(a.A), *W = static_cast<const f16 *>(a.W);
-    auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_blocks * m_blocks)), dim3(kGemmThreads), 0, stream, A,
-                           a.lda, W, a.M, a.N, a.K, a.C, a.ldc, n_blocks, slice_steps);
+    auto go = [&](auto kernel, int groups) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_blocks * m_blocks)), dim3(kGemmThreads * groups), 0, stream,
+                           A, a.lda, W, a.w_packed ? kPackBlock : 32,
+                           a.w_packed ? static_cast<int64_t>(steps) * kPackBlock : int64_t{0}, a.M, a.N, a.K, a.C, a.ldc,
+                           n_blocks, slice_steps);
         return hipGetLastError();
     };
+    if (form == 0) {
+        switch (mt + (ragged ? 1 : 0)) {
+            case 2: return go(gemm_kernel<2, 1, kSplitGroups, EP, false, false>, kSplitGroups);
+            case 3: return go(gemm_kernel<2, 1, kSplitGroups, EP, false, true>, kSplitGroups);
+            case 4: return go(gemm_kernel<4, 1, kSplitGroups, EP, false, false>, kSplitGroups);
+            default: return go(gemm_kernel<4, 1, kSplitGroups, EP, false, true>, kSplitGroups);
+        }
+    }
     switch ((fw == 2 ? 4 : 0) + (ks > 1 ? 2 : 0) + (ragged ? 1 : 0)) {
-        case 0: return go(gemm_kernel<1, EP, false, false>);
-        case 1: return go(gemm_kernel<1, EP, false, true>);
-        case 2: return go(gemm_kernel<1, EP, true, false>);
-        case 3: return go(gemm_kernel<1, EP, true, true>);
-        case 4: return go(gemm_kernel<2, EP, false, false>);
-        case 5: return go(gemm_kernel<2, EP, false, true>);
-        case 6: return go(gemm_kernel<2, EP, true, false>);
-        default: return go(gemm_kernel<2, EP, true, true>);
+        case 0: return go(gemm_kernel<4, 1, 1, EP, false, false>, 1);
+        case 1: return go(gemm_kernel<4, 1, 1, EP, false, true>, 1);
+        case 2: return go(gemm_kernel<4, 1, 1, EP, true, false>, 1);
+        case 3: return go(gemm_kernel<4, 1, 1, EP, true, true>, 1);
+        case 4: return go(gemm_kernel<4, 2, 1, EP, false, false>, 1);
+        case 5: return go(gemm_kernel<4, 2, 1, EP, false, true>, 1);
+        case 6: return go(gemm_kernel<4, 2, 1, EP, true, false>, 1);
+        default: return go(gemm_kernel<4, 2, 1, EP, true, true>, 1);
     }
 }
 
 }  // namespace
 
-// Two feature tiles per wave read A half as often, one gives twice the
-// work-groups: two from 200 work-groups on (us, one against two: 512 x 4096 x
-// 1024, 256 work-groups of two, 10.7 / 10.5; 1800 x 1024 x 2048, 232, 18.1 /
-// 17.8; 256 x 6144 x 1024, 192, 10.4 / 10.9; 512 x 1024 x 2048, 64, 12.3 /
-// 15.4). Four spilled and were within 2% of two.
+// The form by the number of work-groups (us; packed W):
+//  - the split form while its 64 x 64 blocks fit one round at one per CU: its
+//    waves each walk a quarter of K (256 x 1024 x 2048, 64 work-groups, 9.4
+//    against 12.2 with one feature tile per wave and 15.8 with two; 256 x 4096 x
+//    1024, 256, 7.7 / 8.4 / 10.2; 256 x 6144 x 1024, 384, 13.3 / 10.5 / 11.1).
+//    Its LDS reads, 64 rows per feature tile, bound it beyond;
+//  - two feature tiles per wave, which read A half as often, from 200
+//    work-groups on (1800 x 6144 x 1024, one against two, 42.6 / 40.8; 1800 x
+//    1024 x 2048, 232 work-groups, 18.4 / 17.9); up to 64 rows, where W's one
+//    pass is what counts, one (64 x 151936 x 1024 71.8 / 76.6);
+//  - else one. Four feature tiles spilled and were within 2% of two.
+// A row-major W's split form is slower than one tile per wave (48 x 6144 x 2048
+// 14.3 / 12.7).
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
-    const int fw = (a.M + 16 * MT - 1) / (16 * MT) * ((a.N + 127) / 128) >= 200 ? 2 : 1;
+    const int m_blocks = (a.M + 63) / 64;
+    const bool slices = a.workspace && gemv_split(a.N, a.K) > 1;
+    int form = 1;
+    if (a.w_packed && !slices && m_blocks * ((a.N + 63) / 64) <= 256) form = 0;
+    else if (a.M > 64 && m_blocks * ((a.N + 127) / 128) >= 200) form = 2;
     switch (a.epilogue) {
-        case EMBER_EPILOGUE_STORE_F16: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F16>(a, fw, stream);
-        case EMBER_EPILOGUE_STORE_F32: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F32>(a, fw, stream);
-        case EMBER_EPILOGUE_ADD_F32: return launch_gemm_ep<EMBER_EPILOGUE_ADD_F32>(a, fw, stream);
-        case EMBER_EPILOGUE_SILU_MUL: return launch_gemm_ep<EMBER_EPILOGUE_SILU_MUL>(a, fw, stream);
+        case EMBER_EPILOGUE_STORE_F16: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F16>(a, form, stream);
+        case EMBER_EPILOGUE_STORE_F32: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F32>(a, form, stream);
+        case EMBER_EPILOGUE_ADD_F32: return launch_gemm_ep<EMBER_EPILOGUE_ADD_F32>(a, form, stream);
+        case EMBER_EPILOGUE_SILU_MUL: return launch_gemm_ep<EMBER_EPILOGUE_SILU_MUL>(a, form, stream);
         default: return hipErrorInvalidValue;
     }
 }

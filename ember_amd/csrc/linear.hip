@@ -496,10 +496,30 @@ int64_t gemv_workspace(int M, int N, int K) {
     return (nfb * 4 + 255) / 256 * 256 + ks * nfb * mt * 256 * 4;
 }
 
+// Batches of 17 to 64 tokens that the tiled kernel (gemm.hip) serves faster, to
+// the same bits. gemv_kernel's work-groups each read all the activations for 16
+// features: beyond one round of them (N 4096), or with activations too large to
+// stage, that costs more than the tiles' fixed time (us, gemv_kernel against
+// tiles; packed W: 32 x 5120 x 2048 9.6 / 7.4, 17 x 6144 x 1024 5.8 / 5.8, 64 x
+// 4096 x 2048, unstaged, 12.1 / 9.4, 64 x 4096 x 1024, staged, 5.4 / 7.0.
+// Row-major W, whose tiles are slower: 48 x 6144 x 2048 20.1 / 12.7, 32 x 6144 x
+// 2048 12.3 / 12.2, 32 x 12288 x 2048 19.2 / 16.3).
+bool tiles_win(const EmberGemvArgs &a, bool split) {
+    if (split || a.M <= 16) return false;
+    const int64_t stage = static_cast<int64_t>((a.M + 15) / 16) * 16 * a.K * 2;
+    if (a.w_packed) return a.N > 4096 || (a.M > 32 && a.N > 4080 && stage > kGemvMaxStage);
+    return a.M > 32 ? a.N > 4096 : a.N >= 12288;
+}
+
 template <int EP>
 hipError_t launch_gemv_ep(const EmberGemvArgs &a, hipStream_t stream) {
     const int64_t need = gemv_workspace(a.M, a.N, a.K);
     const bool split = need > 0 && a.workspace && a.workspace_bytes >= need;
+    if (tiles_win(a, split)) {
+        EmberGemvArgs t = a;
+        t.workspace = nullptr;
+        return launch_gemm(t, stream);
+    }
     const int nfb = (a.N + 15) / 16;
     const int ks = split ? gemv_split(a.N, a.K) : 1;
     // With fewer 16-feature blocks than kGemvTargetGroups and no K split, each

@@ -775,12 +775,14 @@ def _launch_gemm(g):
 
 
 @pytest.mark.parametrize("M,N,KD", [(65, 48, 32), (127, 130, 96), (128, 4096, 1024), (200, 66, 416), (513, 1024, 3072),
-                                   (100, 2048, 6144), (70, 1040, 4352), (1801, 1024, 2048)])
+                                   (100, 2048, 6144), (70, 1040, 4352), (1801, 1024, 2048), (1000, 1040, 544),
+                                   (1600, 1040, 288)])
 @pytest.mark.parametrize("ep", [0, 1, 2, 3])
 def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
     """More than 64 rows on the tiled kernel: each row is the decode-sized kernel's, bit for bit, with ragged rows and
-    features, k steps that do not divide into the 8 runs (32: empty runs; 416: 13 steps), both tile widths, and the K
-    split's slices (2048 x 6144 over 2; 1040 x 4352 over 2, ragged). Features past N and rows past M stay untouched."""
+    features, k steps that do not divide into the 8 runs (32: empty runs; 416: 13 steps), the form with K groups, both
+    tile widths of the other (1801 rows: two; 1000: one, 17 steps; 1600: two, 9 steps), and the K split's slices (2048 x
+    6144 over 2; 1040 x 4352 over 2, ragged). Features past N and rows past M stay untouched."""
     from ember_amd import _lib
     rng = np.random.default_rng(M + N + KD + ep)
     a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
@@ -798,12 +800,36 @@ def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
         if ws is not None:
             g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
         _launch_gemm(g)
-        for m in range(0, M, 64):
-            n = min(64, M - m)
+        for m in range(0, M, 16):  # up to 16 rows run on the decode-sized kernel at every shape
+            n = min(16, M - m)
             K.gemv(a[m:m + n], w, want[m:m + n], ep, workspace=ws, packed=wp)
         torch.cuda.synchronize()
         view = torch.int32 if f32 else torch.int16
         assert torch.equal(got.view(view), want.view(view)), f"split={ws is not None}"
+
+
+@pytest.mark.parametrize("M,N,KD", [(17, 5120, 2048), (33, 4100, 96), (32, 6144, 1024), (48, 4096, 2048), (64, 12290, 416),
+                                   (20, 12288, 288), (50, 17000, 256)])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("ep", [0, 1, 2, 3])
+def test_gemv_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed, ep):
+    """Batches of 17 to 64 tokens at wide shapes go to the tiled kernel: the same bits as 16 rows at a time, for both W
+    layouts, ragged features, steps that do not divide into the runs, and more blocks than one round."""
+    from ember_amd import _lib
+    rng = np.random.default_rng(M + N + KD + ep)
+    a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
+    w = (torch.randn(N, KD, device=device, generator=torch.Generator(device=device).manual_seed(N)) * 0.05).half()
+    wp = K.gemv_pack(w) if packed else None
+    cols = N // 2 if ep == _lib.EPILOGUE_SILU_MUL else N
+    f32 = ep in (_lib.EPILOGUE_STORE_F32, _lib.EPILOGUE_ADD_F32)
+    got = torch.ones((M, cols), dtype=torch.float32 if f32 else torch.float16, device=device)
+    want = got.clone()
+    K.gemv(a, w, got, ep, packed=wp)
+    for m in range(0, M, 16):
+        K.gemv(a[m:m + 16], w, want[m:m + 16], ep, packed=wp)
+    torch.cuda.synchronize()
+    view = torch.int32 if f32 else torch.int16
+    assert torch.equal(got.view(view), want.view(view))
 
 
 def test_gemv_saturates_f16_outputs(device):
