@@ -320,12 +320,10 @@ private:
 
         for (int l = 0; l < c.n_layers; l++) {
             const LayerWeights &L = layers_[static_cast<size_t>(l)];
-            rmsnorm(nullptr, T, L.in_norm);
-            gemm(xn_.get(), H, L.qkv, T, qkv_.get(), Q + 2 * KV, EMBER_EPILOGUE_STORE_F16);
+            norm_gemm(L.in_norm, L.qkv, T, qkv_.get(), Q + 2 * KV, EMBER_EPILOGUE_STORE_F16);
             kv_->layer(l, qkv_.get(), L.q_norm, L.k_norm, L.qkv_bias, att_.get());
             gemm(att_.get(), Q, L.o, T, h_.get(), H, EMBER_EPILOGUE_ADD_F32);
-            rmsnorm(nullptr, T, L.post_norm);
-            gemm(xn_.get(), H, L.gate_up, T, act_.get(), I, EMBER_EPILOGUE_SILU_MUL);
+            norm_gemm(L.post_norm, L.gate_up, T, act_.get(), I, EMBER_EPILOGUE_SILU_MUL);
             gemm(act_.get(), I, L.down, T, h_.get(), H, EMBER_EPILOGUE_ADD_F32);
             capture(l + 1, T);
         }
@@ -371,9 +369,7 @@ private:
         return true;
     }
 
-    // C[M, N] (+)= A[M, K] . W^T with an epilogue: the decode-sized kernel up to 64 rows, the tiled one beyond
-    // (the same bits per row).
-    void gemm(const void *A, int lda, const Linear &W, int M, void *C, int ldc, int ep) {
+    EmberGemvArgs gemm_args(const void *A, int lda, const Linear &W, int M, void *C, int ldc, int ep) const {
         EmberGemvArgs g{};
         g.A = A;
         g.lda = lda;
@@ -387,6 +383,13 @@ private:
         g.workspace = gemv_ws_.get();
         g.workspace_bytes = static_cast<int64_t>(gemv_ws_.bytes());
         g.w_packed = 1;
+        return g;
+    }
+
+    // C[M, N] (+)= A[M, K] . W^T with an epilogue: the decode-sized kernel up to 64 rows, the tiled one beyond
+    // (the same bits per row).
+    void gemm(const void *A, int lda, const Linear &W, int M, void *C, int ldc, int ep) {
+        const EmberGemvArgs g = gemm_args(A, lda, W, M, C, ldc, ep);
         if (M > 64) {
             HIPB_CHECK(hip::launch_gemm(g, stream_));
         } else {
@@ -394,7 +397,7 @@ private:
         }
     }
 
-    void rmsnorm(const int32_t *rows, int R, const float *w) {
+    EmberNormArgs norm_args(const int32_t *rows, int R, const float *w) const {
         EmberNormArgs n{};
         n.x = h_.get<float>();
         n.rows = rows;
@@ -403,7 +406,24 @@ private:
         n.w = w;
         n.eps = cfg_.rms_eps;
         n.out = xn_.get();
+        return n;
+    }
+
+    void rmsnorm(const int32_t *rows, int R, const float *w) {
+        const EmberNormArgs n = norm_args(rows, R, w);
         check_abi(ember_hip_rmsnorm_rows(&n, stream_), "rmsnorm_rows");
+    }
+
+    // The residual's norm, then a projection of it: one launch where the step is small enough (the same bits).
+    void norm_gemm(const float *w, const Linear &W, int T, void *C, int ldc, int ep) {
+        const EmberNormArgs n = norm_args(nullptr, T, w);
+        const EmberGemvArgs g = gemm_args(xn_.get(), cfg_.hidden, W, T, C, ldc, ep);
+        if (hip::gemv_norm_fits(g, n)) {
+            HIPB_CHECK(hip::launch_gemv_norm(g, n, stream_));
+        } else {
+            rmsnorm(nullptr, T, w);
+            gemm(xn_.get(), cfg_.hidden, W, T, C, ldc, ep);
+        }
     }
 
     void capture(int index, int T) {

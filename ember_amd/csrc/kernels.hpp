@@ -49,6 +49,11 @@ hipError_t launch_gemv_pack(const void *W, int N, int K, void *out, hipStream_t 
 
 hipError_t launch_rmsnorm_rows(const EmberNormArgs &a, hipStream_t stream);
 
+// The norm's rows through the product in one launch (a.A is not read): the
+// bits of launch_rmsnorm_rows followed by launch_gemv. Only where it fits.
+bool gemv_norm_fits(const EmberGemvArgs &a, const EmberNormArgs &n);
+hipError_t launch_gemv_norm(const EmberGemvArgs &a, const EmberNormArgs &n, hipStream_t stream);
+
 hipError_t launch_embed(const EmberEmbedArgs &a, hipStream_t stream);
 hipError_t launch_sample(const EmberSampleArgs &a, hipStream_t stream);
 hipError_t launch_token_probs(const EmberProbArgs &a, hipStream_t stream);

@@ -76,20 +76,32 @@ __device__ __forceinline__ f16x8 load_w(const f16 *p) {
 constexpr int kGemvMaxStage = 128 * 1024;  // bytes of staged activations a work-group may hold
 constexpr int kGemvRedBytes = kGemvWaves * kWave * 16;  // one f32x4 per lane and wave, per 16-token tile
 constexpr int kDescWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
+constexpr int kNormThreads = 256;         // of rmsnorm_rows_kernel
+constexpr int kNormHalf = kNormThreads;   // threads that take one row where the GEMV norms its rows itself
+constexpr int kNormWaves = kNormHalf / kWave;
+constexpr int kNormRows = 8;      // rows it does that for,
+constexpr int kNormFused = 2048;  // and their width at most
 
 // MT tiles of 16 tokens (M <= 16 MT); EP an EMBER_EPILOGUE_*; SPLIT: K split
 // over gridDim.y work-groups (a separate instance, so the unsplit one keeps
 // its constant-stride loads and no merge code). Dynamic LDS: the staged
 // activations (staged) or nothing, and afterwards the waves' partial sums.
-template <int MT, int EP, bool SPLIT, bool PACKED, bool STAGED>
+// NORM: A is the f32 residual, lda its row length, and the staged activations
+// are its RMSNorm (rmsnorm_rows_kernel's arithmetic in its order, so its bits),
+// computed by every work-group for itself: up to kNormRows rows are a few KiB,
+// and the launch of their own that this replaces costs more than the norm.
+template <int MT, int EP, bool SPLIT, bool PACKED, bool STAGED, bool NORM = false>
 __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restrict__ A, int lda,
                                                             const f16 *__restrict__ W, int M, int N, int K,
                                                             void *__restrict__ C, int ldc,
                                                             uint32_t piece_magic, float *__restrict__ slices,
-                                                            uint32_t *__restrict__ counters) {
+                                                            uint32_t *__restrict__ counters,
+                                                            const float *__restrict__ norm_w, float eps) {
+    static_assert(!NORM || (MT == 1 && !SPLIT && PACKED && STAGED));
     extern __shared__ __align__(16) unsigned char gemv_lds[];
     constexpr bool staged = STAGED;
     __shared__ int merge_here;
+    __shared__ double norm_part[NORM ? kNormRows : 1][kNormWaves];
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid % kWave, wave = tid / kWave;
     const int c = lane % 16, g = lane / 16;
@@ -231,10 +243,74 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
+    // NORM: half the work-group's threads take rows 0, 2, ..., the others 1, 3,
+    // ...: thread t of its half elements 4 (t + 256 j) .. + 3, as
+    // rmsnorm_rows_kernel's. The residual is loaded ahead of the round's W, so
+    // the wait for it leaves W in flight.
+    constexpr int kHeld = kNormFused / (4 * kNormHalf), kHalfRows = kNormRows / 2;
+    f32x4 hv[NORM ? kHalfRows : 1][kHeld], nw[kHeld];
+    const int nt = tid % kNormHalf, half = tid / kNormHalf;
+    auto norm_load = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kHeld; j++) {
+            const int i = 4 * (nt + j * kNormHalf);
+#pragma unroll
+            for (int q = 0; q < kHalfRows; q++) {
+                const int r = 2 * q + half;
+                hv[q][j] = r < M && i < K
+                               ? *reinterpret_cast<const f32x4 *>(reinterpret_cast<const float *>(A) + static_cast<int64_t>(r) * lda + i)
+                               : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            nw[j] = i < K ? *reinterpret_cast<const f32x4 *>(norm_w + i) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    };
+    auto norm_stage = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < kHalfRows; q++) {
+            const int r = 2 * q + half;
+            if (r >= M) continue;  // uniform in a wave
+            double ss = 0.0;
+#pragma unroll
+            for (int j = 0; j < kHeld; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) ss += static_cast<double>(hv[q][j][e]) * hv[q][j][e];
+            for (int off = kWave / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+            if (lane == 0) norm_part[r][wave % kNormWaves] = ss;
+        }
+        stage_barrier();
+#pragma unroll
+        for (int q = 0; q < kHalfRows; q++) {
+            const int r = 2 * q + half;
+            if (r >= M) continue;
+            double total = norm_part[r][0];
+            for (int v = 1; v < kNormWaves; v++) total += norm_part[r][v];
+            const float scale = static_cast<float>(1.0 / sqrt(total / K + static_cast<double>(eps)));
+#pragma unroll
+            for (int j = 0; j < kHeld; j++) {
+                const uint32_t i = 4 * (nt + j * kNormHalf);
+                if (static_cast<int>(i) >= K) continue;
+                f16x4 h;
+#pragma unroll
+                for (int e = 0; e < 4; e++) h[e] = static_cast<f16>(clamp_half(nw[j][e] * (hv[q][j][e] * scale)));
+                *reinterpret_cast<f16x4 *>(gemv_lds + 16 * (r * pieces + ((i / 8) ^ (r & 15u))) + 2 * (i % 8)) = h;
+            }
+        }
+        stage_barrier();
+    };
     auto first_round = [&](auto unroll) {
         constexpr int U = decltype(unroll)::value;
         constexpr int E = staged ? (U < gemv_early_w(MT) ? U : gemv_early_w(MT)) : 0;  // W loads ahead of the copies
         f16x8 wv[U];
+        if constexpr (NORM) {
+            norm_load();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < U; u++) wv[u] = load_w(w + wstep * (s + u * stride));
+            __builtin_amdgcn_sched_barrier(0);
+            norm_stage();
+            compute(unroll, wv, s, stride);
+            return;
+        }
 #pragma unroll
         for (int u = 0; u < E; u++) wv[u] = load_w(w + wstep * (s + u * stride));
         __builtin_amdgcn_sched_barrier(0);
@@ -260,7 +336,10 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
         case 2: first_round(std::integral_constant<int, 2>{}); break;
         case 1: first_round(std::integral_constant<int, 1>{}); break;
         default:
-            if constexpr (staged) {
+            if constexpr (NORM) {
+                norm_load();
+                norm_stage();
+            } else if constexpr (staged) {
                 issue_stage();
                 __builtin_amdgcn_s_waitcnt(0);
                 stage_barrier();
@@ -548,7 +627,7 @@ hipError_t launch_gemv_ep(const EmberGemvArgs &a, hipStream_t stream) {
     // raising a per-kernel limit on gfx950 (hipDeviceProp_t::sharedMemPerBlock).
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kGemvThreads), static_cast<unsigned>(lds), stream, A, a.lda, W, a.M, a.N,
-                           a.K, a.C, a.ldc, magic, slices, counters);
+                           a.K, a.C, a.ldc, magic, slices, counters, nullptr, 0.0f);
         return hipGetLastError();
     };
     if (!split && a.M <= 16 && nfb >= kWideMinTiles) {
@@ -612,7 +691,6 @@ __global__ void __launch_bounds__(256) gemv_pack_kernel(const f16 *__restrict__ 
     *reinterpret_cast<f16x8 *>(out + 8 * q) = v;
 }
 
-constexpr int kNormThreads = 256;
 constexpr int kNormPer = 16;  // elements of a row per thread held in registers (hidden <= 4096)
 
 // One work-group per row: the sum of squares in double, reduced in a fixed
@@ -713,6 +791,29 @@ hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream) {
         case EMBER_EPILOGUE_SILU_MUL: return launch_gemv_ep<EMBER_EPILOGUE_SILU_MUL>(a, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+// Decode steps of up to 8 rows, widths up to 2048: the norm's own launch (2.2 us
+// and the gap before the next) costs more than its repetition in every
+// work-group: 1.039 -> 0.927 ms for the 28-layer decode step of one sequence.
+bool gemv_norm_fits(const EmberGemvArgs &a, const EmberNormArgs &n) {
+    return n.R <= kNormRows && n.R == a.M && !n.rows && n.hidden == a.K && a.K <= kNormFused && a.K % 128 == 0 && a.w_packed &&
+           (a.epilogue == EMBER_EPILOGUE_STORE_F16 || a.epilogue == EMBER_EPILOGUE_SILU_MUL) &&
+           (a.N + 15) / 16 < kWideMinTiles &&
+           ((reinterpret_cast<uintptr_t>(n.x) | reinterpret_cast<uintptr_t>(n.w)) & 15) == 0;
+}
+
+hipError_t launch_gemv_norm(const EmberGemvArgs &a, const EmberNormArgs &n, hipStream_t stream) {
+    if (!gemv_norm_fits(a, n)) return hipErrorInvalidValue;
+    const unsigned lds = static_cast<unsigned>(std::max(16 * a.K * 2, kGemvRedBytes));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((a.N + 15) / 16)), dim3(kGemvThreads), lds, stream,
+                           reinterpret_cast<const f16 *>(n.x), n.hidden, static_cast<const f16 *>(a.W), a.M, a.N, a.K, a.C,
+                           a.ldc, 0u, static_cast<float *>(nullptr), static_cast<uint32_t *>(nullptr), n.w, n.eps);
+        return hipGetLastError();
+    };
+    if (a.epilogue == EMBER_EPILOGUE_SILU_MUL) return go(gemv_kernel<1, EMBER_EPILOGUE_SILU_MUL, false, true, true, true>);
+    return go(gemv_kernel<1, EMBER_EPILOGUE_STORE_F16, false, true, true, true>);
 }
 
 hipError_t launch_rmsnorm_rows(const EmberNormArgs &a, hipStream_t stream) {

@@ -452,7 +452,7 @@ struct Dist {
 // nothing settled, when the bound lets too many through.
 __device__ __forceinline__ bool few_candidates(const float *x, int V, const EmberSampleParams &p, float thread_max, Dist &d,
                                SampleLds &sh) {
-    const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave, wave = tid / kWave;
+    const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave;
     const bool by_k = p.top_k > 0 && p.top_k <= kMostCandidates && p.top_k < V;
     const bool by_min_p = !by_k && (p.top_k <= 0 || p.top_k >= V) && !(p.top_p < 1.0f) && d.min_w > 0.0f && d.min_w <= 1.0f;
     if (!by_k && !by_min_p) return false;

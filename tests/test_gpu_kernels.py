@@ -832,6 +832,34 @@ def test_gemv_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed,
     assert torch.equal(got.view(view), want.view(view))
 
 
+@pytest.mark.parametrize("M,N,KD", [(1, 4096, 1024), (2, 48, 128), (3, 6144, 1024), (5, 130, 640), (7, 4100, 1152),
+                                   (8, 12288, 2048)])
+@pytest.mark.parametrize("ep", [0, 3])
+def test_norm_in_the_gemv_equals_two_launches(device, M, N, KD, ep):
+    """The residual's RMSNorm inside the projection's launch: the bits of the norm's own launch and the GEMV's."""
+    import ctypes
+
+    from ember_amd import _lib
+    rng = np.random.default_rng(M + N + KD + ep)
+    h = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float32) * 3).to(device)
+    nw = torch.from_numpy(1 + 0.1 * rng.standard_normal(KD).astype(np.float32)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, KD)) * 0.05).astype(np.float16)).to(device)
+    wp = K.gemv_pack(w)
+    cols = N // 2 if ep == _lib.EPILOGUE_SILU_MUL else N
+    got = torch.ones((M, cols), dtype=torch.float16, device=device)
+    want, xn = got.clone(), torch.empty((M, KD), dtype=torch.float16, device=device)
+    K.rmsnorm_rows(h, nw, xn, 1e-6)
+    K.gemv(xn, w, want, ep, packed=wp)
+    g, n = _lib.GemvArgs(), _lib.NormArgs()
+    g.W, g.M, g.N, g.K, g.C, g.ldc, g.epilogue, g.w_packed = wp.data_ptr(), M, N, KD, got.data_ptr(), cols, ep, 1
+    n.x, n.R, n.hidden, n.w, n.eps = h.data_ptr(), M, KD, nw.data_ptr(), 1e-6
+    fn = _lib.lib()["_ZN5ember3hip16launch_gemv_normERK13EmberGemvArgsRK13EmberNormArgsP12ihipStream_t"]
+    fn.argtypes, fn.restype = [ctypes.c_void_p] * 3, ctypes.c_int
+    assert fn(ctypes.addressof(g), ctypes.addressof(n), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 def test_gemv_saturates_f16_outputs(device):
     """store_f16 clamps to the finite f16 range instead of overflowing to inf (k_gemm.cu's to_half_sat)."""
     a = np.full((2, 64), 100.0, np.float16)
