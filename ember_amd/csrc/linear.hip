@@ -74,6 +74,7 @@ __device__ __forceinline__ f16x8 load_w(const f16 *p) {
 // lanes of a given g hit 16 different slots modulo 16: no bank conflicts.
 // Rows past M read as zeros (offsets past the descriptor's records).
 constexpr int kGemvMaxStage = 128 * 1024;  // bytes of staged activations a work-group may hold
+constexpr int kGemvOwnBytes = kGemvWaves * 16 * 128;     // two k steps of one 16-token tile per wave
 constexpr int kGemvRedBytes = kGemvWaves * kWave * 16;  // one f32x4 per lane and wave, per 16-token tile
 constexpr int kDescWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
 constexpr int kNormThreads = 256;         // of rmsnorm_rows_kernel
@@ -100,6 +101,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     static_assert(!NORM || (MT == 1 && !SPLIT && PACKED && STAGED));
     extern __shared__ __align__(16) unsigned char gemv_lds[];
     constexpr bool staged = STAGED;
+    constexpr bool kOwnStage = SPLIT && !STAGED;
     __shared__ int merge_here;
     __shared__ double norm_part[NORM ? kNormRows : 1][kNormWaves];
     const int tid = static_cast<int>(threadIdx.x);
@@ -327,7 +329,66 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
         }
         compute(unroll, wv, s, stride);
     };
-    const int least = steps / kGemvWaves;
+    // A split launch whose activations are too many to stage: each wave takes
+    // its own run's columns of them through an LDS region of its own, two k
+    // steps at a time, so that memory sees 128 bytes of a row at once (read
+    // straight as operands, 64 from each of 16 rows at a time, the second half
+    // of every line came again after the L1 had lost it; in two slices, 48 x 2048
+    // x 6144 16.1 -> 14.1 us, 64 19.2 -> 15.6). A wave's LDS operations run in order, so no
+    // barrier is needed.
+    if constexpr (kOwnStage) {
+        constexpr int kLoads = 2 * MT;  // 16-byte pieces per lane: row 8 j + lane / 8, piece lane % 8
+        unsigned char *const own = gemv_lds + wave * (MT * 16 * 128);
+        const uint32_t records = static_cast<uint32_t>((static_cast<int64_t>(M - 1) * lda + K) * 2);
+        const __amdgpu_buffer_rsrc_t d = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16 *>(A), 0, records, kDescWord3);
+        uint32_t off[kLoads];
+#pragma unroll
+        for (int j = 0; j < kLoads; j++) {
+            const int r = 8 * j + lane / 8;
+            off[j] = r < M ? static_cast<uint32_t>(r * lda + k0 + 8 * (lane % 8)) * 2u : records;
+        }
+        uint4 av[2][kLoads];
+        f16x8 wv[4];
+        auto load_a = [&](int step, uint4 (&v)[kLoads]) {  // past the records: zeros
+#pragma unroll
+            for (int j = 0; j < kLoads; j++)
+                v[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(d, min(off[j] + 64u * step, records), 0, 0));
+        };
+        const int end = s + left;
+        load_a(s, av[0]);
+#pragma unroll
+        for (int u = 0; u < 4; u++) wv[u] = load_w(w + wstep * min(s + u, steps - 1));
+        load_a(s + 2, av[1]);
+        auto chunk = [&](int i) {
+            if (s >= end) return;
+#pragma unroll
+            for (int j = 0; j < kLoads; j++) {
+                const int r = 8 * j + lane / 8;
+                *reinterpret_cast<uint4 *>(own + 16 * (8 * r + ((lane % 8) ^ (r & 7)))) = av[i][j];
+            }
+            load_a(s + 4, av[i]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+                if (s + v < end) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        const int r = 16 * mt + c;
+                        const f16x8 xv = *reinterpret_cast<const f16x8 *>(own + 16 * (8 * r + ((4 * v + g) ^ (r & 7))));
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[2 * i + v], xv, acc[mt], 0, 0, 0);
+                    }
+                }
+                wv[2 * i + v] = load_w(w + wstep * min(s + v + 4, steps - 1));
+            }
+            s += 2;
+        };
+        while (s < end) {
+            chunk(0);
+            chunk(1);
+        }
+        left = 0;
+    }
+    const int least = kOwnStage ? 0 : steps / kGemvWaves;
     const int first = least >= kGemvUnroll ? kGemvUnroll : min(least, kGemvUnroll / 2);
     switch (first) {
         case kGemvUnroll: first_round(Full{}); break;
@@ -359,7 +420,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     // The waves' partial sums meet in LDS (over the staged activations, once
     // every wave is done with them); wave mt adds token tile mt's in wave order.
     f32x4 *red = reinterpret_cast<f32x4 *>(gemv_lds);  // [wave][mt][lane]
-    if constexpr (staged) __syncthreads();
+    if constexpr (staged || kOwnStage) __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) red[(wave * MT + mt) * kWave + lane] = acc[mt];
     __syncthreads();
@@ -619,7 +680,9 @@ hipError_t launch_gemv_ep(const EmberGemvArgs &a, hipStream_t stream) {
     const int kw = a.K / ks;
     const int stage = 16 * mt * kw * 2;
     const bool staged = kw % 128 == 0 && stage <= kGemvMaxStage;
-    const int lds = staged ? std::max(stage, mt * kGemvRedBytes) : mt * kGemvRedBytes;
+    const int lds = staged ? std::max(stage, mt * kGemvRedBytes)
+                    : split ? mt * kGemvOwnBytes  // each wave's own stage, 2 KiB per token tile
+                            : mt * kGemvRedBytes;
     // ceil(2^32 / pieces): r = t / pieces as one multiply-high for every slot t
     // of the stage (t * pieces < 2^32 since the stage is at most 128 KiB).
     const uint32_t magic = staged ? static_cast<uint32_t>(((uint64_t{1} << 32) + kw / 8 - 1) / (kw / 8)) : 0;
