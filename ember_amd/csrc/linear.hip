@@ -359,6 +359,10 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
 #pragma unroll
         for (int u = 0; u < 4; u++) wv[u] = load_w(w + wstep * min(s + u, steps - 1));
         load_a(s + 2, av[1]);
+        auto own_fence = [] {  // holds the compiler to the order of the lanes' stores and reads; no instruction
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+        };
         auto chunk = [&](int i) {
             if (s >= end) return;
 #pragma unroll
@@ -366,6 +370,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
                 const int r = 8 * j + lane / 8;
                 *reinterpret_cast<uint4 *>(own + 16 * (8 * r + ((lane % 8) ^ (r & 7)))) = av[i][j];
             }
+            own_fence();
             load_a(s + 4, av[i]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -380,6 +385,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
                 }
                 wv[2 * i + v] = load_w(w + wstep * min(s + v + 4, steps - 1));
             }
+            own_fence();
             s += 2;
         };
         while (s < end) {
