@@ -644,17 +644,21 @@ int64_t gemv_workspace(int M, int N, int K) {
 
 // Batches of 17 to 64 tokens that the tiled kernel (gemm.hip) serves faster, to
 // the same bits. gemv_kernel's work-groups each read all the activations for 16
-// features: beyond one round of them (N 4096), or with activations too large to
-// stage, that costs more than the tiles' fixed time (us, gemv_kernel against
-// tiles; packed W: 32 x 5120 x 2048 9.6 / 7.4, 17 x 6144 x 1024 5.8 / 5.8, 64 x
-// 4096 x 2048, unstaged, 12.1 / 9.4, 64 x 4096 x 1024, staged, 5.4 / 7.0.
-// Row-major W, whose tiles are slower: 48 x 6144 x 2048 20.1 / 12.7, 32 x 6144 x
-// 2048 12.3 / 12.2, 32 x 12288 x 2048 19.2 / 16.3).
+// features, which costs more than the tiles' shallower queue of W loads where
+// the activations are too large to stage and there is more than one round of
+// work-groups (N 4096), or where W is large. Measured with W from HBM, as a
+// model's layers have it (us, gemv_kernel against tiles; with weights that the
+// last-level cache holds, the tiles look 1 to 2 us better than they are):
+//  - unstaged: 33 x 5120 x 2048 14.3 / 11.8, 64 rows 21.1 / 13.1; 33 x 4096 x
+//    2048 8.7 / 11.3, 64 rows 11.8 / 12.5; row-major 33 x 12288 x 2048 26.1 / 17.5;
+//  - staged: 32 x 12288 x 2048 15.1 / 14.2, 17 x 151936 x 1024 69 / 62, 64 rows
+//    136 / 73; 32 x 5120 x 2048 8.9 / 10.5, 64 x 6144 x 1024 8.5 / 9.0, 17 rows
+//    5.4 / 7.0; row-major 24 x 12288 x 2048 18.3 / 19.3.
 bool tiles_win(const EmberGemvArgs &a, bool split) {
     if (split || a.M <= 16) return false;
     const int64_t stage = static_cast<int64_t>((a.M + 15) / 16) * 16 * a.K * 2;
-    if (a.w_packed) return a.N > 4096 || (a.M > 32 && a.N > 4080 && stage > kGemvMaxStage);
-    return a.M > 32 ? a.N > 4096 : a.N >= 12288;
+    if (stage > kGemvMaxStage) return a.N > 4096;
+    return a.w_packed && static_cast<int64_t>(a.N) * a.K >= int64_t{12288} * 2048;
 }
 
 template <int EP>

@@ -808,13 +808,14 @@ def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
         assert torch.equal(got.view(view), want.view(view)), f"split={ws is not None}"
 
 
-@pytest.mark.parametrize("M,N,KD", [(17, 5120, 2048), (33, 4100, 96), (32, 6144, 1024), (48, 4096, 2048), (64, 12290, 416),
-                                   (20, 12288, 288), (50, 17000, 256)])
+@pytest.mark.parametrize("M,N,KD", [(17, 12290, 2048), (33, 4100, 1376), (32, 24600, 1024), (48, 4096, 2048), (64, 6144, 2080),
+                                   (20, 90000, 288), (50, 100002, 256)])
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("ep", [0, 1, 2, 3])
 def test_gemv_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed, ep):
-    """Batches of 17 to 64 tokens at wide shapes go to the tiled kernel: the same bits as 16 rows at a time, for both W
-    layouts, ragged features, steps that do not divide into the runs, and more blocks than one round."""
+    """Batches of 17 to 64 tokens whose activations are too large to stage (33 and 64 rows), or whose packed W is large,
+    go to the tiled kernel: the same bits as 16 rows at a time, for both W layouts, ragged features, steps that do not
+    divide into the runs (1376: 43; 288: 9), and more blocks than one round. 4096 features stay with the GEMV."""
     from ember_amd import _lib
     rng = np.random.default_rng(M + N + KD + ep)
     a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
