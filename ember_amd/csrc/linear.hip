@@ -80,7 +80,7 @@ constexpr int kDescWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, 
 constexpr int kNormThreads = 256;         // of rmsnorm_rows_kernel
 constexpr int kNormHalf = kNormThreads;   // threads that take one row where the GEMV norms its rows itself
 constexpr int kNormWaves = kNormHalf / kWave;
-constexpr int kNormRows = 8;      // rows it does that for,
+constexpr int kNormRows = 4;      // rows it does that for,
 constexpr int kNormFused = 2048;  // and their width at most
 
 // MT tiles of 16 tokens (M <= 16 MT); EP an EMBER_EPILOGUE_*; SPLIT: K split
@@ -866,9 +866,10 @@ hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream) {
     }
 }
 
-// Decode steps of up to 8 rows, widths up to 2048: the norm's own launch (2.2 us
+// Decode steps of up to 4 rows, widths up to 2048: the norm's own launch (2.2 us
 // and the gap before the next) costs more than its repetition in every
-// work-group: 1.039 -> 0.927 ms for the 28-layer decode step of one sequence.
+// work-group. The 28-layer decode step, two launches against one: 1 sequence
+// 1.039 / 0.927 ms, 2 1.083 / 0.993, 4 1.175 / 1.125; with 8, 1.351 / 1.415.
 bool gemv_norm_fits(const EmberGemvArgs &a, const EmberNormArgs &n) {
     return n.R <= kNormRows && n.R == a.M && !n.rows && n.hidden == a.K && a.K <= kNormFused && a.K % 128 == 0 && a.w_packed &&
            (a.epilogue == EMBER_EPILOGUE_STORE_F16 || a.epilogue == EMBER_EPILOGUE_SILU_MUL) &&
