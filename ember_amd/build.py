@@ -61,7 +61,7 @@ def common_flags() -> list[str]:
         # No contraction: every multiply-add the kernels fuse is written as fmaf,
         # so rounding is fixed by the source (decode == verify bit-exactly).
         "-ffp-contract=off",
-        # Packed FP32 instructions stay off (they have produced wrong results on this pool).
+        # Packed FP32 instructions stay off (some of their forms have given wrong results on gfx950).
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         f"-I{ROOT / 'include'}",
         f"-I{CSRC}",

@@ -392,7 +392,8 @@ hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, hipStream_t stream) 
 //    work-groups on (1800 x 6144 x 1024, one against two, 42.6 / 40.8; 1800 x
 //    1024 x 2048, 232 work-groups, 18.4 / 17.9); up to 64 rows, where W's one
 //    pass is what counts, one (64 x 151936 x 1024 71.8 / 76.6);
-//  - else one. Four feature tiles spilled and were within 2% of two.
+//  - else one. Four feature tiles spilled and were within 2% of two; 128 tokens
+//    per work-group, at one wave per SIMD, lost (1800 x 4096 x 1024 34.3 / 27.1).
 // A row-major W's split form is slower than one tile per wave (48 x 6144 x 2048
 // 14.3 / 12.7).
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
