@@ -343,10 +343,9 @@ __global__ void __launch_bounds__(kGemmThreads *KG, KG == 1 ? 2 : 1)
     }
 }
 
-// form: 0 the split form, 1 or 2 feature tiles per wave of the other.
+// form: 0 the split form, 1 or 2 feature tiles per wave of the other; ks: K slices (1 with the split form).
 template <int EP>
-hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, hipStream_t stream) {
-    const int ks = form > 0 && a.workspace ? gemv_split(a.N, a.K) : 1;
+hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, int ks, hipStream_t stream) {
     const int steps = a.K / 32, slice_steps = steps / ks;
     const bool ragged = slice_steps % (2 * kLinearRuns * (ks > 1 ? CS : 1)) != 0;  // a run is pairs of chunks
     const int mt = form > 0 || a.M > 32 ? 4 : 2;
@@ -398,15 +397,17 @@ hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, hipStream_t stream) 
 // 14.3 / 12.7).
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
     const int m_blocks = (a.M + 63) / 64;
-    const bool slices = a.workspace && gemv_split(a.N, a.K) > 1;
+    // The sums of a K split only with a workspace that launch_gemv would split with, at its most rows.
+    const bool room = a.workspace && a.workspace_bytes >= gemv_workspace_bytes(64, a.N, a.K);
+    const int ks = room ? gemv_split(a.N, a.K) : 1;
     int form = 1;
-    if (a.w_packed && !slices && m_blocks * ((a.N + 63) / 64) <= 256) form = 0;
+    if (a.w_packed && ks == 1 && m_blocks * ((a.N + 63) / 64) <= 256) form = 0;
     else if (a.M > 64 && m_blocks * ((a.N + 127) / 128) >= 200) form = 2;
     switch (a.epilogue) {
-        case EMBER_EPILOGUE_STORE_F16: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F16>(a, form, stream);
-        case EMBER_EPILOGUE_STORE_F32: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F32>(a, form, stream);
-        case EMBER_EPILOGUE_ADD_F32: return launch_gemm_ep<EMBER_EPILOGUE_ADD_F32>(a, form, stream);
-        case EMBER_EPILOGUE_SILU_MUL: return launch_gemm_ep<EMBER_EPILOGUE_SILU_MUL>(a, form, stream);
+        case EMBER_EPILOGUE_STORE_F16: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F16>(a, form, ks, stream);
+        case EMBER_EPILOGUE_STORE_F32: return launch_gemm_ep<EMBER_EPILOGUE_STORE_F32>(a, form, ks, stream);
+        case EMBER_EPILOGUE_ADD_F32: return launch_gemm_ep<EMBER_EPILOGUE_ADD_F32>(a, form, ks, stream);
+        case EMBER_EPILOGUE_SILU_MUL: return launch_gemm_ep<EMBER_EPILOGUE_SILU_MUL>(a, form, ks, stream);
         default: return hipErrorInvalidValue;
     }
 }

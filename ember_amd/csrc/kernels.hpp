@@ -40,8 +40,8 @@ hipError_t launch_copy_pages(const EmberCopyArgs &a, hipStream_t stream);
 
 hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream);
 // The same product on tiles, for any number of rows: a row's result is the
-// decode-sized kernel's, bit for bit. A workspace (gemv_workspace_bytes of 64
-// rows) means the sums of a K split; it is not written.
+// decode-sized kernel's, bit for bit. A workspace of gemv_workspace_bytes of 64
+// rows or more means the sums of a K split; it is not written.
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream);
 int64_t gemv_workspace_bytes(int M, int N, int K);  // 0: no K split for this shape
 int64_t gemv_packed_bytes(int N, int K);

@@ -808,6 +808,27 @@ def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
         assert torch.equal(got.view(view), want.view(view)), f"split={ws is not None}"
 
 
+def test_gemm_workspace_too_small_for_a_split(device):
+    """A workspace one piece short of 64 rows' is no split, to the tiled kernel as to the GEMV: the unsplit sums' bits."""
+    from ember_amd import _lib
+    M, N, KD = 100, 2048, 6144
+    rng = np.random.default_rng(8)
+    a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, KD)) * 0.05).astype(np.float16)).to(device)
+    wp, ws = K.gemv_pack(w), K.gemv_workspace(64, N, KD, device)
+    got = torch.empty((M, N), dtype=torch.float32, device=device)
+    want = torch.empty_like(got)
+    g = _lib.GemvArgs()
+    g.A, g.lda, g.W, g.M, g.N, g.K = a.data_ptr(), KD, wp.data_ptr(), M, N, KD
+    g.C, g.ldc, g.epilogue, g.w_packed = got.data_ptr(), N, _lib.EPILOGUE_STORE_F32, 1
+    g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel() - 16
+    _launch_gemm(g)
+    K.gemv(a[:64], w, want[:64], _lib.EPILOGUE_STORE_F32, workspace=ws[:-16], packed=wp)
+    K.gemv(a[64:], w, want[64:], _lib.EPILOGUE_STORE_F32, packed=wp)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize("M,N,KD", [(17, 12290, 2048), (33, 4100, 1376), (32, 24600, 1024), (48, 4096, 2048), (64, 6144, 2080),
                                    (20, 90000, 288), (50, 100002, 256)])
 @pytest.mark.parametrize("packed", [False, True])
