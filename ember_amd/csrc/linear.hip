@@ -856,7 +856,27 @@ hipError_t launch_gemv_pack(const void *W, int N, int K, void *out, hipStream_t 
     return hipGetLastError();
 }
 
+// Rows whose A the kernels' 32-bit byte offsets reach (the buffer loads of the
+// stages and the tiles, which run at most a row's width past the last row's start).
+static int rows_in_reach(int lda, int K) {
+    const int64_t halves = (int64_t{1} << 31) - 2 * int64_t{K} - 512;
+    return static_cast<int>(std::clamp<int64_t>(1 + halves / lda, 1, 64));
+}
+
 hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream) {
+    const int most = rows_in_reach(a.lda, a.K);
+    if (a.M > most) {  // rows gigabytes apart: several launches (a row's result does not depend on the batch)
+        const bool f32 = a.epilogue == EMBER_EPILOGUE_STORE_F32 || a.epilogue == EMBER_EPILOGUE_ADD_F32;
+        EmberGemvArgs part = a;
+        if (a.workspace_bytes < gemv_workspace(a.M, a.N, a.K)) part.workspace = nullptr;  // split as one launch would
+        for (int64_t m0 = 0; m0 < a.M; m0 += most) {
+            part.A = static_cast<const f16 *>(a.A) + m0 * a.lda;
+            part.C = static_cast<char *>(a.C) + m0 * a.ldc * (f32 ? 4 : 2);
+            part.M = static_cast<int>(std::min<int64_t>(most, a.M - m0));
+            if (const hipError_t e = launch_gemv(part, stream); e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     switch (a.epilogue) {
         case EMBER_EPILOGUE_STORE_F16: return launch_gemv_ep<EMBER_EPILOGUE_STORE_F16>(a, stream);
         case EMBER_EPILOGUE_STORE_F32: return launch_gemv_ep<EMBER_EPILOGUE_STORE_F32>(a, stream);

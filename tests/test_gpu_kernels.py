@@ -829,6 +829,30 @@ def test_gemm_workspace_too_small_for_a_split(device):
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
 
 
+@pytest.mark.parametrize("M,N,KD,split", [(48, 64, 512, False), (33, 512, 8192, True), (33, 4112, 2048, False), (33, 48, 2080, False)])
+def test_gemv_rows_gigabytes_apart(device, M, N, KD, split):
+    """Rows of A so far apart that the last one starts 4 GiB after the first, as slices of a large buffer: the bits of
+    adjacent rows, with the activations staged, through the waves' own stage, on the tiles, and read directly."""
+    from ember_amd import _lib
+    lda = (1 << 31) // (M - 1) // 8 * 8 + 8
+    a = torch.randn((M, KD), device=device, generator=torch.Generator(device=device).manual_seed(M)).half()
+    w = (torch.randn((N, KD), device=device, generator=torch.Generator(device=device).manual_seed(N)) * 0.05).half()
+    far = torch.empty((M - 1) * lda + KD, dtype=torch.float16, device=device)
+    far.as_strided((M, KD), (lda, 1)).copy_(a)
+    ws = K.gemv_workspace(M, N, KD, device) if split else None
+    got = torch.empty((M, N), dtype=torch.float32, device=device)
+    want = torch.empty_like(got)
+    K.gemv(a, w, want, _lib.EPILOGUE_STORE_F32, workspace=ws)
+    g = _lib.GemvArgs()
+    g.A, g.lda, g.W, g.M, g.N, g.K = far.data_ptr(), lda, w.data_ptr(), M, N, KD
+    g.C, g.ldc, g.epilogue = got.data_ptr(), N, _lib.EPILOGUE_STORE_F32
+    if split:
+        g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
+    _lib.check(_lib.lib().ember_hip_gemv(g, torch.cuda.current_stream().cuda_stream), "gemv")
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
 @pytest.mark.parametrize("M,N,KD", [(17, 12290, 2048), (33, 4100, 1376), (32, 24600, 1024), (48, 4096, 2048), (64, 6144, 2080),
                                    (20, 90000, 288), (50, 100002, 256)])
 @pytest.mark.parametrize("packed", [False, True])
