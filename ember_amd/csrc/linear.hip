@@ -105,7 +105,10 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     __shared__ int merge_here;
     __shared__ double norm_part[NORM ? kNormRows : 1][kNormWaves];
     const int tid = static_cast<int>(threadIdx.x);
-    const int lane = tid % kWave, wave = tid / kWave;
+    // The own stage guards single k steps by the wave's index: as a scalar, so that the guards are branches. An MFMA does
+    // not heed the EXEC mask; a step kept out by a mask alone would be summed. (The rounds below guard none; there a
+    // scalar index moved launches by -3% to +3%, the 16 x 4096 x 1024 one from 3.80 to 3.92 us.)
+    const int lane = tid % kWave, wave = kOwnStage ? __builtin_amdgcn_readfirstlane(tid / kWave) : tid / kWave;
     const int c = lane % 16, g = lane / 16;
     const int fb = static_cast<int>(blockIdx.x), nfb = static_cast<int>(gridDim.x);
     const int ks = SPLIT ? static_cast<int>(blockIdx.y) : 0, KS = SPLIT ? static_cast<int>(gridDim.y) : 1;

@@ -808,6 +808,40 @@ def test_gemm_rows_equal_the_gemv(device, M, N, KD, ep):
         assert torch.equal(got.view(view), want.view(view)), f"split={ws is not None}"
 
 
+@pytest.mark.parametrize("N,KD", [(1040, 4352), (1024, 12288), (1024, 4160), (34, 9216)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_split_gemv_batches_equal_the_tiles(device, N, KD, packed):
+    """Split launches whose activations are too many to stage: each row is the tiled kernel's, bit for bit, for both W
+    layouts. Runs of 8 and 9 steps (4352 in 2 slices of 68 steps), 4 slices (12288), a slice of 65 steps, not a multiple
+    of 128 columns, which no batch stages (4160), and of 72 in 4 slices of runs of 9 (9216); batches that do not fill
+    their 16-row tiles; rows of A further apart than K, with NaN between them."""
+    from ember_amd import _lib
+    rng = np.random.default_rng(N + KD)
+    R, lda = 70, KD + 8
+    wide = torch.full((R, lda), float("nan"), dtype=torch.float16, device=device)
+    wide[:, :KD] = torch.from_numpy(rng.standard_normal((R, KD)).astype(np.float16)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, KD)) * 0.05).astype(np.float16)).to(device)
+    wp, ws = K.gemv_pack(w), K.gemv_workspace(64, N, KD, device)
+
+    def args(M, out, w_packed):
+        g = _lib.GemvArgs()
+        g.A, g.lda, g.W, g.M, g.N, g.K = wide.data_ptr(), lda, (wp if w_packed else w).data_ptr(), M, N, KD
+        g.C, g.ldc, g.epilogue, g.w_packed = out.data_ptr(), N, _lib.EPILOGUE_STORE_F32, int(w_packed)
+        g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
+        return g
+
+    want = torch.empty((R, N), dtype=torch.float32, device=device)
+    _launch_gemm(args(R, want, True))
+    assert _linear_err(want.cpu().numpy(), oracle.linear(wide[:, :KD].contiguous().cpu().numpy(), w.cpu().numpy(),
+                                                         _lib.EPILOGUE_STORE_F32)) < 2e-3
+    for M in (1, 17, 20, 33, 49, 64):
+        got = torch.full((M + 1, N), 7.0, dtype=torch.float32, device=device)
+        _lib.check(_lib.lib().ember_hip_gemv(args(M, got, packed), torch.cuda.current_stream().cuda_stream), "gemv")
+        torch.cuda.synchronize()
+        assert torch.equal(got[:M].view(torch.int32), want[:M].view(torch.int32)), f"M={M}"
+        assert bool((got[M] == 7.0).all()), f"M={M}: a row past the batch"
+
+
 def test_gemm_workspace_too_small_for_a_split(device):
     """A workspace one piece short of 64 rows' is no split, to the tiled kernel as to the GEMV: the unsplit sums' bits."""
     from ember_amd import _lib
