@@ -59,7 +59,7 @@ __device__ __forceinline__ float get_slice(const float *p) {
 }
 
 __device__ __forceinline__ f16x8 load_w(const f16 *p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(p));  // W is read once per launch
+    return __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(p));  // a work-group reads its W once
 }
 
 // Activations staged in LDS (when the launcher passes staged): the
@@ -336,9 +336,12 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     // its own run's columns of them through an LDS region of its own, two k
     // steps at a time, so that memory sees 128 bytes of a row at once (read
     // straight as operands, 64 from each of 16 rows at a time, the second half
-    // of every line came again after the L1 had lost it; in two slices, 48 x 2048
-    // x 6144 16.1 -> 14.1 us, 64 19.2 -> 15.6). A wave's LDS operations run in order, so no
-    // barrier is needed.
+    // of every line came again after the L1 had lost it). The last two chunks
+    // load nothing more: loads past the run cost a launch of runs of 8 to 12
+    // steps what the stage gains (64 x 1024 x 4160, read straight 13.6 us, with
+    // them 14.5, without 10.6). Packed, in two slices, W from HBM: 48 x 2048 x
+    // 6144 15.7 -> 11.5 us, 64 rows 18.9 -> 12.6. A wave's LDS operations run in
+    // order, so no barrier is needed.
     if constexpr (kOwnStage) {
         constexpr int kLoads = 2 * MT;  // 16-byte pieces per lane: row 8 j + lane / 8, piece lane % 8
         unsigned char *const own = gemv_lds + wave * (MT * 16 * 128);
@@ -360,13 +363,14 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
         const int end = s + left;
         load_a(s, av[0]);
 #pragma unroll
-        for (int u = 0; u < 4; u++) wv[u] = load_w(w + wstep * min(s + u, steps - 1));
-        load_a(s + 2, av[1]);
+        for (int u = 0; u < 4; u++) wv[u] = load_w(w + wstep * min(s + u, end - 1));
+        load_a(min(s + 2, end - 1), av[1]);
         auto own_fence = [] {  // holds the compiler to the order of the lanes' stores and reads; no instruction
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
         };
-        auto chunk = [&](int i) {
+        // Chunk i of a pair, steps s and s + 1 (if it is in the run); with its registers' next loads, or without.
+        auto chunk = [&](auto more, int i) {
             if (s >= end) return;
 #pragma unroll
             for (int j = 0; j < kLoads; j++) {
@@ -374,7 +378,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
                 *reinterpret_cast<uint4 *>(own + 16 * (8 * r + ((lane % 8) ^ (r & 7)))) = av[i][j];
             }
             own_fence();
-            load_a(s + 4, av[i]);
+            if constexpr (decltype(more)::value) load_a(min(s + 4, end - 1), av[i]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int v = 0; v < 2; v++) {
@@ -386,15 +390,17 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
                         acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wv[2 * i + v], xv, acc[mt], 0, 0, 0);
                     }
                 }
-                wv[2 * i + v] = load_w(w + wstep * min(s + v + 4, steps - 1));
+                if constexpr (decltype(more)::value) wv[2 * i + v] = load_w(w + wstep * min(s + v + 4, end - 1));
             }
             own_fence();
             s += 2;
         };
-        while (s < end) {
-            chunk(0);
-            chunk(1);
+        while (s + 4 < end) {
+            chunk(std::true_type{}, 0);
+            chunk(std::true_type{}, 1);
         }
+        chunk(std::false_type{}, 0);
+        chunk(std::false_type{}, 1);
         left = 0;
     }
     const int least = kOwnStage ? 0 : steps / kGemvWaves;
