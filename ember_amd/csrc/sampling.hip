@@ -12,7 +12,9 @@
 // min_p. The token is argmax over the kept set of v + Gumbel noise (the Gumbel-max trick,
 // sampling_rng.hpp:20-33: the noise depends only on (seed, counter, token id),
 // so a row draws the same token in any batch). Greedy rows (temperature <=
-// 1e-5) take the first largest logit.
+// 1e-5) take the first largest logit. Rows whose largest v is not finite have no
+// masses to cut by; they take the first largest v, as the host's draw does (a
+// +inf logit wins over any noise; token 0 when all are -inf or NaN).
 //
 // What bounds it: passes of one CU over the row (608 KB at 151,936 logits, 6 to
 // 10 us each), so the cuts are found in few of them. All sums are integers
@@ -370,8 +372,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
                                           float top_p, unsigned long long &kept, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
     const bool prob = top_p >= 0.0f;
-    // (mx - v) rounds the same way for equal v and never orders two v the other way round, so bins follow the order
-    // (with an infinite mx, every element is in the last one).
+    // (mx - v) rounds the same way for equal v and never orders two v the other way round, so bins follow the order.
     auto bin_of = [&](float v) {
         const float d = (mx - v) * kBinsPerUnit;
         return d < static_cast<float>(kBins - 1) ? static_cast<int>(d) : kBins - 1;
@@ -397,9 +398,8 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
     }
     __syncthreads();
     kept = total;
-    const bool none = prob && total == 0;  // an infinite maximum: nothing has weight, which the radix search settles
-    if (total < target && !none) return within;
-    const int bin = none ? kBins : static_cast<int>(sh.prefix);
+    if (total < target) return within;
+    const int bin = static_cast<int>(sh.prefix);
     const unsigned long long above = sh.above;
     for_row(x, V, [&](int i, float xi) {
         const float v = xi / t;
@@ -410,7 +410,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
     __syncthreads();
     const int n = sh.listed;
     Cut c;
-    if (n <= kList && !none) {
+    if (n <= kList) {
         sort_list(n, sh);
         const unsigned long long e0 = 2 * tid < n ? sh.list[2 * tid] : 0, e1 = 2 * tid + 1 < n ? sh.list[2 * tid + 1] : 0;
         const unsigned long long w0 = 2 * tid < n ? (prob ? fixed_weight(entry_value(e0), mx) : 1ull) : 0;
@@ -438,6 +438,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
 
 struct Dist {
     bool greedy;
+    bool certain;  // the largest v is not finite: nothing below it is settled
     float t, mx, min_w;
     Cut k, p;              // the top-k and top-p cuts (the top-p one lies inside the top-k one)
     unsigned long long z;  // fixed-point mass of the kept set (where asked for)
@@ -523,11 +524,13 @@ __device__ __forceinline__ Dist distribution(const float *x, int V, const EmberS
     float m = -INFINITY;
     for_row(x, V, [&](int, float xi) { m = fmaxf(m, xi); });
     d.mx = block_max(m, sh) / d.t;  // the largest quotient: division by t > 0 keeps the order
+    d.certain = !(fabsf(d.mx) < INFINITY);
+    if (d.certain) return d;
     d.min_w = p.min_p > 0.0f ? p.min_p : 0.0f;
     const Cut all;
     d.k = all;
     d.p = all;
-    if (fabsf(d.mx) < INFINITY && d.t < 1e5f && few_candidates(x, V, p, m, d, sh)) return d;
+    if (d.t < 1e5f && few_candidates(x, V, p, m, d, sh)) return d;
     unsigned long long kept = 0;  // weight of the set so far
     bool known = false;           // and it is the kept set's mass
 #pragma unroll 1
@@ -567,6 +570,8 @@ __global__ void __launch_bounds__(kSampleThreads) sample_kernel(const float *__r
     int tok;
     if (d.greedy) {
         tok = block_argmax(x, V, [](int, float xi) { return xi; }, sh);
+    } else if (d.certain) {
+        tok = block_argmax(x, V, [&](int, float xi) { return xi / d.t; }, sh);
     } else if (d.listed) {
         float best = -INFINITY;
         int idx = 0x7fffffff;
@@ -606,6 +611,8 @@ __global__ void __launch_bounds__(kSampleThreads) prob_kernel(const float *__res
     float prob;
     if (d.greedy) {
         prob = block_argmax(x, V, [](int, float xi) { return xi; }, sh) == tok ? 1.0f : 0.0f;
+    } else if (d.certain) {  // 0 for every token of a row with nothing above -inf
+        prob = block_argmax(x, V, [&](int, float xi) { return xi / d.t; }, sh) == tok && d.mx > 0.0f ? 1.0f : 0.0f;
     } else {
         const float v = scaled(x, tok, d.t);
         const float w = expf(v - d.mx);

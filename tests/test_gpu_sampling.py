@@ -198,3 +198,28 @@ def test_rows_with_infinities_and_nan():
     assert gpu_sample(np.tile(x, (4, 1)), forms) == gpu_sample(np.tile(clean, (4, 1)), forms)
     everything = np.full(5000, -np.inf, np.float32)  # nothing to choose from: token 0, as for a greedy row of NaN
     assert gpu_sample(np.tile(everything, (4, 1)), forms) == [0] * 4
+
+
+@pytest.mark.parametrize("V", [40, 5000])
+def test_rows_whose_largest_quotient_is_infinite(V):
+    """One or more +inf logits, or finite ones that the temperature divides past the f32 range, beside ordinary, -inf and
+    NaN ones: the host's draw under every cut, the first of them, whose probability is 1 and every other token's 0."""
+    rng = np.random.default_rng(V)
+    one, two, far = (rng.normal(0.0, 2.0, V).astype(np.float32) for _ in range(3))
+    one[V // 2] = np.inf
+    two[[V - 3, 11, V // 3]] = np.inf
+    two[[2, 20]] = -np.inf
+    far[[V - 2, 9]] = 3e38, 2e38  # 2e38 / 0.5 is past the range too: equal, the lower id first
+    cuts = [(1.0, 0, 0.0), (1.0, 5, 0.0), (0.9, 0, 0.0), (0.9, 30, 0.0), (1.0, 0, 0.05), (0.9, 30, 0.05), (1.0, V - 1, 0.0)]
+    for x, first, other in ((one, V // 2, 0), (two, 11, V // 3), (far, 9, V - 2)):
+        rows = [(0.5, top_p, top_k, min_p, 3, c) for c, (top_p, top_k, min_p) in enumerate(cuts)]
+        want = [oracle.sample(x, *r[:4], seed=r[4], counter=r[5]) for r in rows]
+        assert want == [first] * len(rows)
+        assert gpu_sample(np.tile(x, (len(rows), 1)), rows) == want
+        queries = [(r, tok) for r in range(len(rows)) for tok in (first, other, 1)]
+        assert gpu_probs(np.tile(x, (len(rows), 1)), rows, queries).tolist() == [1.0, 0.0, 0.0] * len(rows)
+    one[7] = np.nan  # never drawn, and nothing beside it changes
+    assert gpu_sample(np.tile(one, (len(rows), 1)), rows) == [V // 2] * len(rows)
+    nothing = np.full(V, -np.inf, np.float32)
+    assert gpu_sample(np.tile(nothing, (len(rows), 1)), rows) == [0] * len(rows)
+    assert gpu_probs(np.tile(nothing, (len(rows), 1)), rows, [(r, 0) for r in range(len(rows))]).tolist() == [0.0] * len(rows)
