@@ -21,16 +21,20 @@
 // (counts, and exp(v - max) in 2^-40 fixed point), so they are the same
 // whatever order the LDS atomics land in, and the kept set is a deterministic
 // function of the logits (float atomics would make it depend on scheduling at
-// the boundary). Three ways, the first that applies:
+// the boundary). Two ways, the first that applies:
 //  - candidates: a lower bound of the k-th largest logit from the threads'
 //    maxima (one pass), then the few elements at or above it are collected,
 //    sorted in LDS, and every cut, the mass and the draw come from that list;
 //  - bins: a histogram over 1/64-wide steps below the maximum (one pass), then
-//    the elements of the one bin that the cut falls in are collected and sorted;
-//  - radix: 8 bits per pass over order-preserving uint32 keys of v, for bins
-//    that hold more elements than the list.
+//    the elements of the one bin that the cut falls in are collected and sorted.
+//    While they are more than the list holds and differ, their range of keys
+//    (order-preserving uint32 of v) is split into as many bins again; a tie's
+//    cut is then found by radix over the ids.
 // 16 rows of 151,936, top-k 40 and top-p 0.9: sample 27 us (303 by radix alone),
 // token_probs 25 us (276); top-p 0.95 alone, by bins: 133 us (289) and 92 (248).
+// Sample, masked to 30 tokens, top-k 40 and top-p 0.9: 107 us (1042); 80 distinct
+// logits, top-p 0.95: 303 (523); all equal: 485 (1046), most of it in passes
+// whose atomics all go to one bin.
 #include <cstdint>
 
 #include "device.hpp"
@@ -76,17 +80,18 @@ struct SampleLds {
     float wmax[kSampleWaves];
     int widx[kSampleWaves];
     uint32_t prefix, mask;
-    unsigned long long above, at;  // after a selection: the weight above the found key, and at it
+    unsigned long long above;  // after a selection: the weight (or count) before what it found
     unsigned long long bins[kBins];
     unsigned long long list[kList];  // elements as (key of v, ~id): descending is the order of the cuts
     int listed;
+    uint32_t low, high;  // the keys of a bin's last and first elements
 };
 
 // A prefix of the (v descending, id ascending) order.
 struct Cut {
     float theta = -INFINITY;
     int id_cut = 0x7fffffff;
-    __device__ bool keeps(float v, int i) const { return v > theta || (v == theta && i <= id_cut); }
+    __device__ __forceinline__ bool keeps(float v, int i) const { return v > theta || (v == theta && i <= id_cut); }
 };
 
 __device__ __forceinline__ float scaled(const float *x, int i, float t) { return x[i] / t; }
@@ -172,7 +177,7 @@ __device__ __forceinline__ int entry_id(unsigned long long e) { return static_ca
 
 // Sorts sh.list[0, n) descending, n <= kList; every thread calls it. Entries
 // past n are overwritten with 0, which orders after every entry.
-__device__ void sort_list(int n, SampleLds &sh) {
+__device__ __forceinline__ void sort_list(int n, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
     int size = 2;
     while (size < n) size *= 2;
@@ -194,7 +199,7 @@ __device__ void sort_list(int n, SampleLds &sh) {
 }
 
 // The index of the threads' largest best (ties to the lowest; 0 if none is above -inf).
-__device__ int block_first_largest(float best, int idx, SampleLds &sh) {
+__device__ __forceinline__ int block_first_largest(float best, int idx, SampleLds &sh) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         const float ob = __shfl_xor(best, o, kWave);
@@ -223,7 +228,7 @@ __device__ int block_first_largest(float best, int idx, SampleLds &sh) {
 
 // First largest score(i, x[i]) over i < V (ties to the lowest index).
 template <class F>
-__device__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
+__device__ __forceinline__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
     float best = -INFINITY;
     int idx = 0x7fffffff;
     for_row(x, V, [&](int i, float xi) {
@@ -234,64 +239,6 @@ __device__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
         }
     });
     return block_first_largest(best, idx, sh);
-}
-
-// The largest key K such that the weight of the elements with key >= K (among
-// those `within` keeps) reaches `target`; weight 1 (prob = false) or
-// exp(v - mx) in fixed point (prob = true). Returns the value of K; sh.above
-// and sh.at then hold the weight above K and at K.
-__device__ __forceinline__ float radix_threshold(const float *x, int V, float t, const Cut within, float mx, bool prob,
-                                 unsigned long long target, SampleLds &sh) {
-    const int tid = static_cast<int>(threadIdx.x);
-    if (tid == 0) {
-        sh.prefix = 0;
-        sh.mask = 0;
-        sh.above = 0;
-    }
-    for (int shift = 24; shift >= 0; shift -= 8) {
-        for (int i = tid; i < 256; i += kSampleThreads) sh.hist[i] = 0;
-        __syncthreads();
-        const uint32_t prefix = sh.prefix, mask = sh.mask;
-        for_row(x, V, [&](int i, float xi) {
-            const float v = xi / t;
-            if (!within.keeps(v, i)) return;
-            const uint32_t k = order_key(v);
-            if ((k & mask) != prefix) return;
-            atomicAdd(&sh.hist[(k >> shift) & 255u], prob ? fixed_weight(v, mx) : 1ull);
-        });
-        __syncthreads();
-        if (tid < kWave) {  // wave 0 finds the digit: lane l holds bins 255 - 4l .. 252 - 4l
-            unsigned long long mine = 0;
-            for (int j = 0; j < 4; j++) mine += sh.hist[255 - 4 * tid - j];
-            // inclusive scan from the top bins down (lane 0 first)
-            unsigned long long incl = mine;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const unsigned long long up = __shfl_up(incl, o, kWave);
-                if (tid >= o) incl += up;
-            }
-            const unsigned long long above = sh.above;
-            const unsigned long long before = incl - mine;  // weight of the higher lanes' bins
-            // the first lane whose cumulative weight reaches the target (or the last lane)
-            const bool hit = above + incl >= target;
-            const unsigned long long ballot = __ballot(hit);
-            const int first = ballot ? __ffsll(static_cast<long long>(ballot)) - 1 : kWave - 1;
-            if (tid == first) {
-                unsigned long long cum = above + before;
-                int d = 255 - 4 * tid;
-                for (int j = 0; j < 3; j++, d--) {
-                    if (cum + sh.hist[d] >= target) break;
-                    cum += sh.hist[d];
-                }
-                sh.above = cum;
-                sh.at = sh.hist[d];
-                sh.prefix = prefix | (static_cast<uint32_t>(d) << shift);
-                sh.mask = mask | (255u << shift);
-            }
-        }
-        __syncthreads();
-    }
-    return key_value(sh.prefix);
 }
 
 // The r-th lowest id (r >= 1) among the elements `within` keeps whose v equals
@@ -305,7 +252,7 @@ __device__ __forceinline__ int kth_tied_id(const float *x, int V, float t, const
         sh.mask = 0;
         sh.above = 0;  // here: the count below the bins looked at so far
     }
-    for (int shift = 24; shift >= 0; shift -= 8) {
+    for (int shift = V > 1 ? (31 - __clz(V - 1)) / 8 * 8 : 0; shift >= 0; shift -= 8) {  // ids below V have no higher bytes
         for (int i = tid; i < 256; i += kSampleThreads) sh.hist[i] = 0;
         __syncthreads();
         const uint32_t prefix = sh.prefix, mask = sh.mask;
@@ -345,76 +292,129 @@ __device__ __forceinline__ int kth_tied_id(const float *x, int V, float t, const
     return static_cast<int>(sh.prefix);
 }
 
-// The cut at the key radix_threshold just found (in sh): when the weight at
-// that key holds more tied tokens than the target still needs, only the lowest
-// ids that reach it are kept. w_each: the weight of one token at the key.
-__device__ __forceinline__ Cut cut_at(const float *x, int V, float t, const Cut within, float theta, unsigned long long target,
-                      unsigned long long w_each, SampleLds &sh) {
-    Cut c;
-    c.theta = theta;
-    const unsigned long long above = sh.above, at = sh.at;
-    __syncthreads();  // every thread has read sh before it is reused
-    if (w_each == 0 || target <= above) return c;
-    const unsigned long long need = (target - above + w_each - 1) / w_each, ties = at / w_each;
-    if (need < ties) c.id_cut = kth_tied_id(x, V, t, within, theta, need, sh);
-    return c;
-}
-
 __device__ __forceinline__ unsigned long long top_p_target(float top_p, unsigned long long mass) {
     const double want = ceil(static_cast<double>(top_p) * static_cast<double>(mass));
     return want < 1.0 ? 1ull : static_cast<unsigned long long>(want);
 }
 
-// The prefix of `within` (in the cuts' order) whose weight first reaches the
-// target: `top_k` elements (top_p < 0), or top_p of the mass of `within`.
-// `kept`: the prefix's weight.
-__device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const Cut within, float mx, int top_k,
-                                          float top_p, unsigned long long &kept, SampleLds &sh) {
+// The first bin, from 0 up, at which the sums of sh.bins and `above` reach the
+// target (set from the sum of all where target_of says so): true, with sh.prefix
+// the bin and sh.above the weight before it, or false if they never do.
+template <class F>
+__device__ __forceinline__ bool find_bin(unsigned long long above, F target_of, unsigned long long &total, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
-    const bool prob = top_p >= 0.0f;
-    // (mx - v) rounds the same way for equal v and never orders two v the other way round, so bins follow the order.
-    auto bin_of = [&](float v) {
-        const float d = (mx - v) * kBinsPerUnit;
-        return d < static_cast<float>(kBins - 1) ? static_cast<int>(d) : kBins - 1;
-    };
-    __syncthreads();
-    for (int i = tid; i < kBins; i += kSampleThreads) sh.bins[i] = 0;
-    if (tid == 0) sh.listed = 0;
-    __syncthreads();
-    for_row(x, V, [&](int i, float xi) {
-        const float v = xi / t;
-        if (!within.keeps(v, i)) return;
-        const unsigned long long w = prob ? fixed_weight(v, mx) : 1ull;
-        if (w) atomicAdd(&sh.bins[bin_of(v)], w);
-    });
-    __syncthreads();
     const unsigned long long b0 = sh.bins[2 * tid], b1 = sh.bins[2 * tid + 1];
-    unsigned long long total;
-    const unsigned long long before = block_scan_u64(b0 + b1, sh, total);
-    const unsigned long long target = prob ? top_p_target(top_p, total) : static_cast<unsigned long long>(top_k);
-    if (before < target && before + b0 + b1 >= target) {  // one thread (none if the total falls short)
+    const unsigned long long before = above + block_scan_u64(b0 + b1, sh, total), target = target_of(total);
+    if (before < target && before + b0 + b1 >= target) {  // one thread at most
         sh.prefix = static_cast<uint32_t>(2 * tid + (before + b0 >= target ? 0 : 1));
         sh.above = before + (before + b0 >= target ? 0 : b0);
     }
     __syncthreads();
-    kept = total;
-    if (total < target) return within;
-    const int bin = static_cast<int>(sh.prefix);
-    const unsigned long long above = sh.above;
-    for_row(x, V, [&](int i, float xi) {
-        const float v = xi / t;
-        if (!within.keeps(v, i) || bin_of(v) != bin) return;
-        const int at = atomicAdd(&sh.listed, 1);
-        if (at < kList) sh.list[at] = list_entry(v, i);
-    });
-    __syncthreads();
-    const int n = sh.listed;
+    return above + total >= target;
+}
+
+// The prefix of `within` (in the cuts' order) whose weight first reaches the
+// target: `top_k` elements (top_p < 0), or top_p of the mass of `within`; all of
+// it if it holds less. `kept`: the prefix's weight. Elements of -inf, which have
+// no mass and are never drawn, are not counted: a row masked to fewer than top_k
+// tokens keeps them all and looks for no cut among the rest.
+__device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const Cut within, float mx, int top_k,
+                                          float top_p, unsigned long long &kept, SampleLds &sh) {
+    const int tid = static_cast<int>(threadIdx.x);
+    const bool prob = top_p >= 0.0f;
+    auto weight = [&](float v) { return prob ? fixed_weight(v, mx) : 1ull; };
+    // The sums of bin_of(v)'s bins over the elements of `within` above -inf (bin < 0: left out).
+    auto fill_bins = [&](auto bin_of) {
+        __syncthreads();
+        for (int i = tid; i < kBins; i += kSampleThreads) sh.bins[i] = 0;
+        __syncthreads();
+        for_row(x, V, [&](int i, float xi) {
+            const float v = xi / t;
+            if (!(v > -INFINITY)) return;
+            const int b = bin_of(v);
+            if (b < 0 || !within.keeps(v, i)) return;
+            const unsigned long long w = weight(v);
+            if (w) atomicAdd(&sh.bins[b], w);
+        });
+        __syncthreads();
+    };
+    // The elements of `within` above -inf that in(v) takes, into sh.list: how many they are and, where the list does not
+    // hold them, their lowest and highest key.
+    uint32_t low = 0, high = 0;
+    auto collect = [&](auto in) {
+        if (tid == 0) {
+            sh.listed = 0;
+            sh.low = ~0u;
+            sh.high = 0;
+        }
+        __syncthreads();
+        low = ~0u;
+        high = 0;
+        for_row(x, V, [&](int i, float xi) {
+            const float v = xi / t;
+            if (!(v > -INFINITY) || !in(v) || !within.keeps(v, i)) return;
+            const int at = atomicAdd(&sh.listed, 1);
+            if (at < kList) sh.list[at] = list_entry(v, i);
+            low = min(low, order_key(v));
+            high = max(high, order_key(v));
+        });
+        __syncthreads();
+        const int found = sh.listed;
+        if (found > kList) {
+#pragma unroll
+            for (int o = kWave / 2; o > 0; o >>= 1) {
+                low = min(low, static_cast<uint32_t>(__shfl_xor(static_cast<int>(low), o, kWave)));
+                high = max(high, static_cast<uint32_t>(__shfl_xor(static_cast<int>(high), o, kWave)));
+            }
+            if (tid % kWave == 0) {
+                atomicMin(&sh.low, low);
+                atomicMax(&sh.high, high);
+            }
+            __syncthreads();
+            low = sh.low;
+            high = sh.high;
+        }
+        return found;
+    };
+
+    // (mx - v) rounds the same way for equal v and never orders two v the other way round, so bins follow the order.
+    auto step_of = [&](float v) {
+        const float d = (mx - v) * kBinsPerUnit;
+        return d < static_cast<float>(kBins - 1) ? static_cast<int>(d) : kBins - 1;
+    };
+    fill_bins(step_of);
+    unsigned long long target = 0;
+    auto set_target = [&](unsigned long long total) {
+        return target = prob ? top_p_target(top_p, total) : static_cast<unsigned long long>(top_k);
+    };
+    if (!find_bin(0, set_target, kept, sh)) return within;
+    const int step = static_cast<int>(sh.prefix);
+    unsigned long long above = sh.above;
+    int n = collect([&](float v) { return step_of(v) == step; });
+#pragma unroll 1
+    while (n > kList && low < high) {  // at most three times: 32 bits of key, 11 of them a time
+        const int shift = max(0, 32 - __clz(static_cast<int>(high - low)) - 11);  // (high - low) >> shift < kBins
+        const uint32_t lo = low, hi = high;
+        fill_bins([&](float v) {
+            const uint32_t k = order_key(v) - lo;
+            return k > hi - lo ? -1 : kBins - 1 - static_cast<int>(k >> shift);
+        });
+        unsigned long long sum;
+        find_bin(above, [&](unsigned long long) { return target; }, sum, sh);
+        const uint32_t part = static_cast<uint32_t>(kBins - 1) - sh.prefix;
+        above = sh.above;
+        __syncthreads();  // every thread has read sh before it is reused
+        n = collect([&](float v) {
+            const uint32_t k = order_key(v) - lo;
+            return k <= hi - lo && k >> shift == part;
+        });
+    }
     Cut c;
     if (n <= kList) {
         sort_list(n, sh);
         const unsigned long long e0 = 2 * tid < n ? sh.list[2 * tid] : 0, e1 = 2 * tid + 1 < n ? sh.list[2 * tid + 1] : 0;
-        const unsigned long long w0 = 2 * tid < n ? (prob ? fixed_weight(entry_value(e0), mx) : 1ull) : 0;
-        const unsigned long long w1 = 2 * tid + 1 < n ? (prob ? fixed_weight(entry_value(e1), mx) : 1ull) : 0;
+        const unsigned long long w0 = 2 * tid < n ? weight(entry_value(e0)) : 0;
+        const unsigned long long w1 = 2 * tid + 1 < n ? weight(entry_value(e1)) : 0;
         unsigned long long all;
         const unsigned long long pre = above + block_scan_u64(w0 + w1, sh, all);
         __syncthreads();
@@ -429,11 +429,12 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
         kept = sh.above;
         return c;
     }
-    const float theta = radix_threshold(x, V, t, within, mx, prob, target, sh);
-    const unsigned long long w_each = prob ? fixed_weight(theta, mx) : 1ull, over = sh.above, at = sh.at;
-    const unsigned long long need = w_each == 0 || target <= over ? 0 : (target - over + w_each - 1) / w_each;
-    kept = over + (need && need * w_each < at ? need * w_each : at);
-    return cut_at(x, V, t, within, theta, target, w_each, sh);
+    // One value, more often than the list holds: the lowest ids of the tie, as many as reach the target.
+    const unsigned long long each = weight(key_value(high)), need = (target - above + each - 1) / each;
+    c.theta = key_value(high);
+    if (need < static_cast<unsigned long long>(n)) c.id_cut = kth_tied_id(x, V, t, within, c.theta, need, sh);
+    kept = above + min(need, static_cast<unsigned long long>(n)) * each;
+    return c;
 }
 
 struct Dist {
@@ -443,7 +444,7 @@ struct Dist {
     Cut k, p;              // the top-k and top-p cuts (the top-p one lies inside the top-k one)
     unsigned long long z;  // fixed-point mass of the kept set (where asked for)
     int listed;            // the kept set is within sh.list[0, listed), sorted; 0: not listed
-    __device__ bool keeps(float v, int i) const { return k.keeps(v, i) && p.keeps(v, i) && expf(v - mx) >= min_w; }
+    __device__ __forceinline__ bool keeps(float v, int i) const { return k.keeps(v, i) && p.keeps(v, i) && expf(v - mx) >= min_w; }
 };
 
 // Rows whose kept set is among few elements: those at or above a bound that

@@ -200,6 +200,43 @@ def test_rows_with_infinities_and_nan():
     assert gpu_sample(np.tile(everything, (4, 1)), forms) == [0] * 4
 
 
+def _few_values(kind, V, rng):
+    if kind == "equal":
+        return np.full(V, 1.25, np.float32)
+    if kind == "steps":  # about a dozen values: every bin holds more than a list
+        return np.round(rng.normal(0.0, 1.0, V) * 2).astype(np.float32) / 2
+    low = {"masked to -inf": -np.inf, "masked to the lowest": np.finfo(np.float32).min, "masked to -1e4": -1e4}[kind]
+    x = np.full(V, low, np.float32)
+    x[rng.choice(V, 12, replace=False)] = rng.normal(0.0, 2.0, 12)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["equal", "steps", "masked to -inf", "masked to the lowest", "masked to -1e4"])
+@pytest.mark.parametrize("V", [3000, 151936])
+def test_rows_of_few_distinct_values(kind, V):
+    """Cuts inside runs of thousands of equal logits, found by radix in one bin, and top-k beyond the tokens a mask
+    allows: the host's kept set, its probabilities either side of the cut, and its draws."""
+    rng = np.random.default_rng(V + len(kind))
+    x = _few_values(kind, V, rng)
+    forms = [(0.8, 0.9, 40, 0.0), (1.0, 1.0, 5, 0.0), (0.9, 1.0, 600, 0.0), (0.9, 0.7, 2500, 0.0), (1.0, 0.95, 0, 0.0),
+             (1.0, 0.95, 0, 0.3), (0.7, 1.0, 0, 0.05), (1.3, 0.5, 0, 0.0), (0.9, 1.0, V - 1, 0.0)]
+    rows, queries, want = [], [], []
+    for i, (t, top_p, top_k, min_p) in enumerate(forms):
+        kept, probs = oracle.sampling_distribution(x, t, top_p, top_k, min_p)
+        rows.append((t, top_p, top_k, min_p, 55, 0))
+        inside = {int(tok): p for tok, p in zip(kept, probs)}
+        order = np.argsort(-x, kind="stable")
+        for tok in {*order[:2], *order[max(0, len(kept) - 2):len(kept) + 2]}:
+            queries.append((i, int(tok)))
+            want.append(inside.get(int(tok), 0.0))
+    got = gpu_probs(np.tile(x, (len(forms), 1)), rows, queries)
+    # a kept set of n equal weights sums n values of 2^-40 fixed point on the GPU, n doubles on the host
+    np.testing.assert_allclose(got, np.array(want, np.float32), rtol=1e-4, atol=1e-12)
+    draws = [r[:5] + (c,) for r in rows for c in range(3)]
+    toks = gpu_sample(np.tile(x, (len(draws), 1)), draws)
+    assert toks == [oracle.sample(x, *r[:4], seed=r[4], counter=r[5]) for r in draws]
+
+
 @pytest.mark.parametrize("V", [40, 5000])
 def test_rows_whose_largest_quotient_is_infinite(V):
     """One or more +inf logits, or finite ones that the temperature divides past the f32 range, beside ordinary, -inf and
