@@ -200,6 +200,28 @@ def test_rows_with_infinities_and_nan():
     assert gpu_sample(np.tile(everything, (4, 1)), forms) == [0] * 4
 
 
+@pytest.mark.parametrize("V", [40, 1030, 8192, 151936])
+@pytest.mark.parametrize("kind", ["flat", "peaked", "masked"])
+def test_min_p_alone_and_no_cut(kind, V):
+    """Probabilities of the tokens either side of a min-p cut, few or more than the list holds, and without any cut, are
+    the host's; the draws from the unordered list too."""
+    rng = np.random.default_rng(V)
+    x = _row(kind, V, rng)
+    forms = [(1.0, 1.0, 0, 0.0), (1.2, 1.0, 0, 0.02), (0.7, 1.0, 0, 0.3), (1.0, 1.0, 0, 1.0), (1.1, 1.0, V, 1e-6)]
+    queries, want = [], []
+    for i, (t, top_p, top_k, min_p) in enumerate(forms):
+        kept, probs = oracle.sampling_distribution(x, t, top_p, top_k, min_p)
+        left = np.setdiff1d(np.argsort(-x, kind="stable")[:len(kept) + 3], kept)
+        for tok, p in [*zip(kept[:3], probs[:3]), *zip(kept[-3:], probs[-3:]), *((tok, 0.0) for tok in left)]:
+            queries.append((i, int(tok)))
+            want.append(p)
+    rows = [(*f, 5, 0) for f in forms]
+    np.testing.assert_allclose(gpu_probs(np.tile(x, (len(forms), 1)), rows, queries), np.array(want, np.float32),
+                               rtol=2e-4, atol=1e-9)
+    draws = [(*f, 5, c) for f in forms for c in range(4)]
+    assert gpu_sample(np.tile(x, (len(draws), 1)), draws) == [oracle.sample(x, *r[:4], seed=5, counter=r[5]) for r in draws]
+
+
 def _few_values(kind, V, rng):
     if kind == "equal":
         return np.full(V, 1.25, np.float32)
