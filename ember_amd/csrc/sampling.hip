@@ -72,7 +72,10 @@ __device__ __forceinline__ float gumbel_noise(uint64_t seed, uint64_t counter, u
 constexpr int kList = 2 * kSampleThreads;  // elements a cut's list holds
 constexpr int kBins = 2 * kSampleThreads;  // of 1 / kBinsPerUnit each, below the largest scaled logit
 constexpr float kBinsPerUnit = 64.0f;
-constexpr int kMostCandidates = 512;  // the largest top-k whose candidates are looked for
+// The largest top-k whose candidates are looked for: 512, where a pass over the row costs more than sorting the 1000 or
+// so that they are (16 rows of 151,936, top-k 512: 45 us, by bins 115); in short rows less (token_probs of 4 rows of
+// 8192, top-k 512: 19 to 23 us, by bins 19, before either 20; top-k 200: 16.4, 18.5).
+__device__ __forceinline__ int most_candidates(int V) { return max(128, min(512, V / 32)); }
 
 struct SampleLds {
     unsigned long long hist[256];
@@ -184,6 +187,8 @@ __device__ __forceinline__ void sort_list(int n, SampleLds &sh) {
     __syncthreads();
     for (int i = n + tid; i < size; i += kSampleThreads) sh.list[i] = 0;
     __syncthreads();
+    // Up to j = 64 a wave's pairs lie within its own 128 entries, and its LDS operations run in order: a barrier only
+    // before and after steps that reach further. (One after each of the 66 steps of 2048 entries: 3 us more.)
     for (int k = 2; k <= size; k *= 2)
         for (int j = k / 2; j > 0; j /= 2) {
             if (tid < size / 2) {  // pair (i, i + j); kList / 2 threads at most
@@ -194,8 +199,15 @@ __device__ __forceinline__ void sort_list(int n, SampleLds &sh) {
                     sh.list[i + j] = a;
                 }
             }
-            __syncthreads();
+            const int next = j > 1 ? j / 2 : k;
+            if (max(j, next) > kWave) {
+                __syncthreads();
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
+    __syncthreads();
 }
 
 // The index of the threads' largest best (ties to the lowest; 0 if none is above -inf).
@@ -456,7 +468,7 @@ struct Dist {
 __device__ __forceinline__ bool few_candidates(const float *x, int V, const EmberSampleParams &p, float thread_max, bool cuts,
                                                Dist &d, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x), lane = tid % kWave;
-    const bool by_k = p.top_k > 0 && p.top_k <= kMostCandidates && p.top_k < V;
+    const bool by_k = p.top_k > 0 && p.top_k <= most_candidates(V) && p.top_k < V;
     if (!by_k && (cuts || !(d.least > -INFINITY))) return false;
     float bound;
     if (by_k) {
