@@ -39,6 +39,8 @@ int prefill_attn(const EmberPrefillArgs *a, hipStream_t stream, hipEvent_t start
 hipError_t launch_copy_pages(const EmberCopyArgs &a, hipStream_t stream);
 
 hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream);
+// Batches of 17 to 64 tokens that launch_gemv gives to the tiles (launch_gemm): the same bits, faster.
+bool gemv_on_tiles(const EmberGemvArgs &a, bool split);
 // The same product on tiles, for any number of rows: a row's result is the
 // decode-sized kernel's, bit for bit. A workspace of gemv_workspace_bytes of 64
 // rows or more means the sums of a K split; it is not written.

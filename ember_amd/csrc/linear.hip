@@ -640,6 +640,30 @@ int gemv_split(int N, int K) {
     return ks;
 }
 
+// gemv_kernel's work-groups each read all the activations for 16 features, which
+// costs more than the tiles' shallower queue of W loads where there are many
+// features or the activations are too large to stage. Time by the tiles over
+// time by gemv_kernel, W from HBM, as a model's layers have it (with weights that
+// the last-level cache holds, the tiles look 1 to 2 us better than they are):
+//  - staged: packed, 12288 x 2048 0.84 to 0.91, 24576 x 1024 0.92 to 0.99, 151936 x
+//    1024 0.9 up to 32 rows, 0.55 at 64; but 6144 x 1024 1.06 to 1.3, 5120 x 2048
+//    1.18, row-major 12288 x 2048 1.0. (65536 x 1024, 17 to 24 rows: 1.05 to 1.1.)
+//  - unstaged, more than 8192 features (over two work-groups per CU): K 1376 to 8192,
+//    17 rows 0.82 to 1.0, 32 rows 0.65 to 0.8, 64 rows 0.45 to 0.75, both W layouts;
+//  - unstaged, 4112 to 8192 features: packed, 17 rows 1.05 to 1.2, 24 rows 0.93 to
+//    1.06, 32 rows 0.85 to 0.95, 64 rows 0.63 to 0.7; row-major, 32 rows 0.98 to 1.12,
+//    33 rows 0.87 to 1.07, 40 rows 0.8 to 1.0. Rows that are not whole 128-byte lines
+//    (K 1376, 2080) spread over the L1's sets: gemv_kernel reads them faster, 33 rows 1.1
+//    to 1.3, 49 rows 0.92 to 1.1;
+//  - unstaged, 4096 features, one round of work-groups: 33 x 4096 x 2048 1.3, 64 rows 1.06.
+bool gemv_on_tiles(const EmberGemvArgs &a, bool split) {
+    if (split || a.M <= 16 || a.M > 64) return false;
+    const int64_t stage = static_cast<int64_t>((a.M + 15) / 16) * 16 * a.K * 2;
+    if (stage <= kGemvMaxStage) return a.w_packed && static_cast<int64_t>(a.N) * a.K >= int64_t{12288} * 2048;
+    if (a.N > 8192) return true;
+    return a.N > 4096 && a.lda % 64 == 0 && a.K % 64 == 0 && a.M > (a.w_packed ? 24 : 36);
+}
+
 namespace {
 
 // Workspace of a split launch: the merge counters (one per 16 features,
@@ -651,30 +675,11 @@ int64_t gemv_workspace(int M, int N, int K) {
     return (nfb * 4 + 255) / 256 * 256 + ks * nfb * mt * 256 * 4;
 }
 
-// Batches of 17 to 64 tokens that the tiled kernel (gemm.hip) serves faster, to
-// the same bits. gemv_kernel's work-groups each read all the activations for 16
-// features, which costs more than the tiles' shallower queue of W loads where
-// the activations are too large to stage and there is more than one round of
-// work-groups (N 4096), or where W is large. Measured with W from HBM, as a
-// model's layers have it (us, gemv_kernel against tiles; with weights that the
-// last-level cache holds, the tiles look 1 to 2 us better than they are):
-//  - unstaged: 33 x 5120 x 2048 14.3 / 11.8, 64 rows 21.1 / 13.1; 33 x 4096 x
-//    2048 8.7 / 11.3, 64 rows 11.8 / 12.5; row-major 33 x 12288 x 2048 26.1 / 17.5;
-//  - staged: 32 x 12288 x 2048 15.1 / 14.2, 17 x 151936 x 1024 69 / 62, 64 rows
-//    136 / 73; 32 x 5120 x 2048 8.9 / 10.5, 64 x 6144 x 1024 8.5 / 9.0, 17 rows
-//    5.4 / 7.0; row-major 24 x 12288 x 2048 18.3 / 19.3.
-bool tiles_win(const EmberGemvArgs &a, bool split) {
-    if (split || a.M <= 16) return false;
-    const int64_t stage = static_cast<int64_t>((a.M + 15) / 16) * 16 * a.K * 2;
-    if (stage > kGemvMaxStage) return a.N > 4096;
-    return a.w_packed && static_cast<int64_t>(a.N) * a.K >= int64_t{12288} * 2048;
-}
-
 template <int EP>
 hipError_t launch_gemv_ep(const EmberGemvArgs &a, hipStream_t stream) {
     const int64_t need = gemv_workspace(a.M, a.N, a.K);
     const bool split = need > 0 && a.workspace && a.workspace_bytes >= need;
-    if (tiles_win(a, split)) {
+    if (gemv_on_tiles(a, split)) {
         EmberGemvArgs t = a;
         t.workspace = nullptr;
         return launch_gemm(t, stream);

@@ -912,6 +912,58 @@ def test_gemv_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed,
     assert torch.equal(got.view(view), want.view(view))
 
 
+@pytest.mark.parametrize("M,N,KD", [(20, 9730, 2080), (31, 16400, 2112), (26, 4114, 2240), (40, 4112, 2112), (64, 8192, 2176),
+                                   (40, 9728, 1376)])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("ep", [1, 3])
+def test_unstaged_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed, ep):
+    """Batches too large to stage, over the tiled kernel's instances for them: packed, four K groups over 32-row blocks
+    with runs that are not whole pairs of chunks (20 rows, 65 steps) and 64-row blocks of both kinds (40 rows: 66 and 43
+    steps; 64: 68), one K group (16400 features); row-major, one K group. 26 rows go to the tiles packed only."""
+    from ember_amd import _lib
+    rng = np.random.default_rng(M + N + KD + ep)
+    a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
+    w = (torch.randn(N, KD, device=device, generator=torch.Generator(device=device).manual_seed(N)) * 0.05).half()
+    wp = K.gemv_pack(w) if packed else None
+    cols = N // 2 if ep == _lib.EPILOGUE_SILU_MUL else N
+    f32 = ep == _lib.EPILOGUE_STORE_F32
+    got = torch.ones((M, cols), dtype=torch.float32 if f32 else torch.float16, device=device)
+    want = got.clone()
+    K.gemv(a, w, got, ep, packed=wp)
+    for m in range(0, M, 16):
+        K.gemv(a[m:m + 16], w, want[m:m + 16], ep, packed=wp)
+    torch.cuda.synchronize()
+    view = torch.int32 if f32 else torch.int16
+    assert torch.equal(got.view(view), want.view(view))
+
+
+@pytest.mark.parametrize("M,N,KD", [(801, 2048, 6144), (1500, 1040, 4352)])
+@pytest.mark.parametrize("ep", [1, 2, 3])
+def test_sliced_gemm_of_two_tiles_per_wave(device, M, N, KD, ep):
+    """The K split's slices with two feature tiles per wave (200 work-groups of them or more), runs of whole chunk pairs
+    (12 steps) and not (8 and 9), against the split GEMV's rows."""
+    from ember_amd import _lib
+    rng = np.random.default_rng(M + N + KD + ep)
+    a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, KD)) * 0.05).astype(np.float16)).to(device)
+    wp, ws = K.gemv_pack(w), K.gemv_workspace(64, N, KD, device)
+    cols = N // 2 if ep == _lib.EPILOGUE_SILU_MUL else N
+    f32 = ep in (_lib.EPILOGUE_STORE_F32, _lib.EPILOGUE_ADD_F32)
+    start = torch.from_numpy(rng.standard_normal((M, cols)).astype(np.float32)).to(device)
+    got = start.clone() if f32 else start.half()
+    want = got.clone()
+    g = _lib.GemvArgs()
+    g.A, g.lda, g.W, g.M, g.N, g.K = a.data_ptr(), KD, wp.data_ptr(), M, N, KD
+    g.C, g.ldc, g.epilogue, g.w_packed = got.data_ptr(), cols, ep, 1
+    g.workspace, g.workspace_bytes = ws.data_ptr(), ws.numel()
+    _launch_gemm(g)
+    for m in range(0, M, 16):
+        K.gemv(a[m:m + 16], w, want[m:m + 16], ep, workspace=ws, packed=wp)
+    torch.cuda.synchronize()
+    view = torch.int32 if f32 else torch.int16
+    assert torch.equal(got.view(view), want.view(view))
+
+
 @pytest.mark.parametrize("M,N,KD", [(1, 4096, 1024), (2, 48, 128), (3, 6144, 1024), (3, 130, 640), (4, 4100, 1152),
                                    (4, 12288, 2048)])
 @pytest.mark.parametrize("ep", [0, 3])

@@ -1,0 +1,46 @@
+"""Which kernel a linear layer's launch takes, by its sizes. The choices are host code in the library and need no GPU;
+every kernel gives a row the same bits (test_gpu_kernels.py), so only the time depends on them. Each line of a table was
+measured on both sides, W from HBM."""
+import pytest
+
+from ember_amd import _lib
+
+
+def _gemv_args(M, N, K, packed, lda=None):
+    g = _lib.GemvArgs()
+    g.M, g.N, g.K, g.lda, g.ldc, g.w_packed = M, N, K, lda or K, N, int(packed)
+    return g
+
+
+def _host(symbol, restype, *argtypes):
+    fn = _lib.lib()[symbol]
+    fn.restype, fn.argtypes = restype, list(argtypes)
+    return fn
+
+
+@pytest.mark.parametrize("M,N,K,packed,tiles", [
+    # up to 16 rows, and one round of work-groups: the decode-sized kernel
+    (16, 151936, 1024, True, False), (16, 24576, 4096, False, False), (64, 4096, 2048, True, False),
+    (33, 4096, 2048, False, False),
+    # staged activations: tiles for large packed W only
+    (32, 12288, 2048, True, True), (17, 151936, 1024, True, True), (64, 151936, 1024, True, True),
+    (64, 6144, 1024, True, False), (32, 5120, 2048, True, False), (32, 12288, 2048, False, False),
+    # too many to stage, more than 8192 features: tiles for either layout (17 x 9728 x 2560, row-major: 22.5 -> 20.6 us)
+    (17, 9728, 2560, False, True), (17, 9728, 2560, True, True), (33, 9728, 1376, False, True),
+    # up to 8192: few rows and row-major W stay (us, GEMV against tiles: 17 x 6144 x 2560, row-major, 15.5 / 19.6; 24 x
+    # 5120 x 2560 16.8 / 19.8; 17 x 8192 x 3072, packed, 14.7 / 16.5)
+    (17, 6144, 2560, False, False), (24, 5120, 2560, False, False), (32, 8192, 4096, False, False),
+    (17, 8192, 3072, True, False), (20, 8192, 3072, True, False),
+    (32, 4112, 4096, True, True), (33, 4112, 2560, True, True), (40, 4112, 2560, False, True),
+    # rows of A that are not whole 128-byte lines (us: 33 x 4112 x 2080, packed, 11.2 / 12.9)
+    (33, 4112, 2080, True, False), (64, 5000, 1376, True, False), (33, 5000, 2080, False, False),
+])
+def test_batches_of_17_to_64_on_tiles(M, N, K, packed, tiles):
+    import ctypes
+    fn = _host("_ZN5ember3hip13gemv_on_tilesERK13EmberGemvArgsb", ctypes.c_bool, ctypes.c_void_p, ctypes.c_bool)
+    g = _gemv_args(M, N, K, packed)
+    assert fn(ctypes.addressof(g), False) is tiles
+    assert fn(ctypes.addressof(g), True) is False  # a K split stays
+    if tiles and N <= 8192:
+        g.lda = K + 32
+        assert fn(ctypes.addressof(g), False) is False
