@@ -251,7 +251,8 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_kernel(const f16 *__restric
     // NORM: half the work-group's threads take rows 0, 2, ..., the others 1, 3,
     // ...: thread t of its half elements 4 (t + 256 j) .. + 3, as
     // rmsnorm_rows_kernel's. The residual is loaded ahead of the round's W, so
-    // the wait for it leaves W in flight.
+    // the wait for it leaves W in flight. Rows from M up of the stage are left as
+    // they are: an operand row reaches its own token's outputs only.
     constexpr int kHeld = kNormFused / (4 * kNormHalf), kHalfRows = kNormRows / 2;
     f32x4 hv[NORM ? kHalfRows : 1][kHeld], nw[kHeld];
     const int nt = tid % kNormHalf, half = tid / kNormHalf;
@@ -903,11 +904,20 @@ hipError_t launch_gemv(const EmberGemvArgs &a, hipStream_t stream) {
 // Decode steps of up to 4 rows, widths up to 2048: the norm's own launch (2.2 us
 // and the gap before the next) costs more than its repetition in every
 // work-group. The 28-layer decode step, two launches against one: 1 sequence
-// 1.039 / 0.927 ms, 2 1.083 / 0.993, 4 1.175 / 1.125; with 8, 1.351 / 1.415.
+// 1.039 / 0.927 ms, 2 1.083 / 0.993, 4 1.175 / 1.101; with 8, 1.351 / 1.415.
+// It is repeated in every round of work-groups, so the more there are, the longer
+// a work-group's W must take to hide it. One launch's time over two's: up to 512
+// work-groups (two per CU) 0.6 to 0.9, 4 rows 0.7 to 0.99 (8192 x 128, 4 rows: 1.02);
+// up to 1024, K 512: 0.8 to 0.94 with 1 or 2 rows, 1.01 to 1.07 with 3, 1.2 with 4;
+// K 1024: 0.87 to 0.99 up to 3 rows, 1.01 to 1.05 with 4; K 2048: 0.82 to 0.99;
+// beyond: 20480 x 1024, 2 rows 1.04, 4 rows 1.14.
 bool gemv_norm_fits(const EmberGemvArgs &a, const EmberNormArgs &n) {
-    return n.R <= kNormRows && n.R == a.M && !n.rows && n.hidden == a.K && a.K <= kNormFused && a.K % 128 == 0 && a.w_packed &&
-           (a.epilogue == EMBER_EPILOGUE_STORE_F16 || a.epilogue == EMBER_EPILOGUE_SILU_MUL) &&
-           (a.N + 15) / 16 < kWideMinTiles &&
+    if (n.R < 1 || n.R > kNormRows) return false;
+    const int groups = (a.N + 15) / 16;
+    const bool pays = groups <= 256 || (groups <= 512 && a.K >= 64 * n.R) ||
+                      (groups <= 1024 && a.K >= 512 << std::max(0, n.R - 2));
+    return n.R == a.M && !n.rows && n.hidden == a.K && a.K <= kNormFused && a.K % 128 == 0 && a.w_packed &&
+           (a.epilogue == EMBER_EPILOGUE_STORE_F16 || a.epilogue == EMBER_EPILOGUE_SILU_MUL) && pays &&
            ((reinterpret_cast<uintptr_t>(n.x) | reinterpret_cast<uintptr_t>(n.w)) & 15) == 0;
 }
 

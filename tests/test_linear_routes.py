@@ -1,6 +1,8 @@
 """Which kernel a linear layer's launch takes, by its sizes. The choices are host code in the library and need no GPU;
 every kernel gives a row the same bits (test_gpu_kernels.py), so only the time depends on them. Each line of a table was
 measured on both sides, W from HBM."""
+import ctypes
+
 import pytest
 
 from ember_amd import _lib
@@ -36,7 +38,6 @@ def _host(symbol, restype, *argtypes):
     (33, 4112, 2080, True, False), (64, 5000, 1376, True, False), (33, 5000, 2080, False, False),
 ])
 def test_batches_of_17_to_64_on_tiles(M, N, K, packed, tiles):
-    import ctypes
     fn = _host("_ZN5ember3hip13gemv_on_tilesERK13EmberGemvArgsb", ctypes.c_bool, ctypes.c_void_p, ctypes.c_bool)
     g = _gemv_args(M, N, K, packed)
     assert fn(ctypes.addressof(g), False) is tiles
@@ -44,3 +45,23 @@ def test_batches_of_17_to_64_on_tiles(M, N, K, packed, tiles):
     if tiles and N <= 8192:
         g.lda = K + 32
         assert fn(ctypes.addressof(g), False) is False
+
+
+@pytest.mark.parametrize("R,N,K,one", [
+    # up to 512 work-groups: one launch (us, two launches against one: 4 x 4096 x 1024 5.7 / 4.2, 4 x 8192 x 2048 0.96)
+    (1, 4096, 1024, True), (4, 6144, 1024, True), (4, 8192, 2048, True), (4, 2048, 128, True), (5, 4096, 1024, False),
+    (4, 8192, 128, False), (1, 4096, 2176, False),
+    # up to 1024: where W takes long enough to hide the repeated norm (4 x 12288 x 512 6.6 / 7.8)
+    (4, 12288, 2048, True), (1, 12288, 512, True), (2, 16384, 512, True), (3, 16384, 1024, True),
+    (3, 12288, 512, False), (4, 12288, 512, False), (4, 12288, 1024, False), (4, 12288, 1536, False), (2, 16384, 128, False),
+    # beyond: two (4 x 65520 x 1024 25.3 / 35.6)
+    (1, 16400, 2048, False), (4, 65520, 1024, False),
+])
+def test_the_norm_inside_the_projection(R, N, K, one):
+    fn = _host("_ZN5ember3hip14gemv_norm_fitsERK13EmberGemvArgsRK13EmberNormArgs", ctypes.c_bool, ctypes.c_void_p,
+               ctypes.c_void_p)
+    g, n = _gemv_args(R, N, K, True), _lib.NormArgs()
+    n.R, n.hidden = R, K
+    assert fn(ctypes.addressof(g), ctypes.addressof(n)) is one
+    g.w_packed = 0
+    assert fn(ctypes.addressof(g), ctypes.addressof(n)) is False
