@@ -343,6 +343,12 @@ __global__ void __launch_bounds__(kGemmThreads *KG, KG == 1 ? 2 : 1)
     }
 }
 
+// K slices: only with a workspace that launch_gemv would split with, at its most rows.
+int slices(const EmberGemvArgs &a) {
+    const bool room = a.workspace && a.workspace_bytes >= gemv_workspace_bytes(64, a.N, a.K);
+    return room ? gemv_split(a.N, a.K) : 1;
+}
+
 // form: 0 the split form, 1 or 2 feature tiles per wave of the other; ks: K slices (1 with the split form).
 template <int EP>
 hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, int ks, hipStream_t stream) {
@@ -381,6 +387,24 @@ hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, int ks, hipStream_t 
 
 }  // namespace
 
+// 65 to 128 rows of few features: two launches of the decode-sized kernel, whose
+// work-groups are more (per 16 features and 16 tokens, or K slice) and each walk
+// less of K. Time by the tiles over theirs, packed, W from HBM: up to 1024
+// features, K 256 to 4096, 1.2 to 1.7; up to 2048 features, K 256 to 1024, 1.03
+// to 1.26, in K slices (K above 4096) 1.26 to 3; K 2048, up to 1536 features, 1.01 to
+// 1.18, 2048 features 1.03 to 1.06 up to 96 rows, 0.94 beyond; K 3072 and 4096 0.75
+// to 1.0 (1280 features 0.84 to 1.14); 2560 and 3072 features, K 256 and 512, 1.02 to 1.19
+// up to 96 rows, K 1024 0.79 to 0.98; 4080 features 0.4 to 0.9. From 129 rows on the tiles win
+// unsplit (129 x 1024 x 2048 11.9 / 10.5), three launches against one.
+bool gemm_by_gemv(const EmberGemvArgs &a) {
+    if (a.M <= 64 || a.M > 128) return false;
+    const bool split = slices(a) > 1;
+    if (a.N <= 1024) return split || a.K <= 4096;
+    if (a.N <= 1536) return split || a.K <= 2048;
+    if (a.N <= 2048) return split || a.K <= 1024 || (a.K <= 2048 && a.M <= 96);
+    return a.N <= 3072 && a.K <= 512 && a.M <= 96;
+}
+
 // The form by the number of work-groups (us; packed W):
 //  - the split form while its 64 x 64 blocks fit one round at one per CU: its
 //    waves each walk a quarter of K (256 x 1024 x 2048, 64 work-groups, 9.4
@@ -397,9 +421,7 @@ hipError_t launch_gemm_ep(const EmberGemvArgs &a, int form, int ks, hipStream_t 
 // 14.3 / 12.7).
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
     const int m_blocks = (a.M + 63) / 64;
-    // The sums of a K split only with a workspace that launch_gemv would split with, at its most rows.
-    const bool room = a.workspace && a.workspace_bytes >= gemv_workspace_bytes(64, a.N, a.K);
-    const int ks = room ? gemv_split(a.N, a.K) : 1;
+    const int ks = slices(a);
     int form = 1;
     if (a.w_packed && ks == 1 && m_blocks * ((a.N + 63) / 64) <= 256) form = 0;
     else if (a.M > 64 && m_blocks * ((a.N + 127) / 128) >= 200) form = 2;

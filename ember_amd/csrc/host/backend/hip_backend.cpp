@@ -386,13 +386,19 @@ private:
         return g;
     }
 
-    // C[M, N] (+)= A[M, K] . W^T with an epilogue: the decode-sized kernel up to 64 rows, the tiled one beyond
-    // (the same bits per row).
+    // C[M, N] (+)= A[M, K] . W^T with an epilogue: the decode-sized kernel up to 64 rows, the tiled one or two launches
+    // of the decode-sized one beyond (the same bits per row).
     void gemm(const void *A, int lda, const Linear &W, int M, void *C, int ldc, int ep) {
-        const EmberGemvArgs g = gemm_args(A, lda, W, M, C, ldc, ep);
-        if (M > 64) {
+        EmberGemvArgs g = gemm_args(A, lda, W, M, C, ldc, ep);
+        if (M > 64 && !hip::gemm_by_gemv(g)) {
             HIPB_CHECK(hip::launch_gemm(g, stream_));
-        } else {
+            return;
+        }
+        const size_t out_elem = ep == EMBER_EPILOGUE_STORE_F32 || ep == EMBER_EPILOGUE_ADD_F32 ? 4 : 2;
+        for (int m0 = 0; m0 < M; m0 += 64) {
+            g.A = static_cast<const char *>(A) + static_cast<size_t>(m0) * lda * 2;
+            g.C = static_cast<char *>(C) + static_cast<size_t>(m0) * ldc * out_elem;
+            g.M = std::min(64, M - m0);
             check_abi(ember_hip_gemv(&g, stream_), "gemv");
         }
     }

@@ -45,6 +45,8 @@ bool gemv_on_tiles(const EmberGemvArgs &a, bool split);
 // decode-sized kernel's, bit for bit. A workspace of gemv_workspace_bytes of 64
 // rows or more means the sums of a K split; it is not written.
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream);
+// Products of 65 to 128 rows that two launches of launch_gemv, 64 rows and the rest, do faster, to the same bits.
+bool gemm_by_gemv(const EmberGemvArgs &a);
 int64_t gemv_workspace_bytes(int M, int N, int K);  // 0: no K split for this shape
 int64_t gemv_packed_bytes(int N, int K);
 hipError_t launch_gemv_pack(const void *W, int N, int K, void *out, hipStream_t stream);

@@ -98,6 +98,16 @@ def test_uneven_chunks_at_block_offset_3(model):
     be.close()
 
 
+def test_chunks_of_65_to_128_tokens(model):
+    """Steps whose qkv and gate/up run on the tiled kernel and whose o and down run 64 rows at a time: 65, 100 and 128
+    tokens, and 129, where all are on tiles."""
+    d, w = model
+    be = create_backend(str(d), BackendOptions(max_batch_tokens=512, max_seqs=8, kv_cache_tokens=64 * PAGE))
+    worst, _ = _greedy_run(be, OracleModel(w), [65, 100, 128, 129], 1, 0, np.random.default_rng(8))
+    assert worst < 2e-2, f"logits differ from the oracle by {worst:.2e}"
+    be.close()
+
+
 def test_capture_hidden_and_token_probs(model):
     d, w = model
     be = create_backend(str(d), BackendOptions(max_batch_tokens=64, max_seqs=4, kv_cache_tokens=8 * PAGE))

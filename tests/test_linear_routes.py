@@ -65,3 +65,23 @@ def test_the_norm_inside_the_projection(R, N, K, one):
     assert fn(ctypes.addressof(g), ctypes.addressof(n)) is one
     g.w_packed = 0
     assert fn(ctypes.addressof(g), ctypes.addressof(n)) is False
+
+
+@pytest.mark.parametrize("M,N,K,split,gemv", [
+    # us, W from HBM, tiles against two launches: 65 x 1024 x 2048 10.5 / 7.8, 128 x 1024 x 3072 16.0 / 10.9
+    (65, 1024, 2048, False, True), (128, 1024, 3072, False, True), (128, 512, 1024, False, True),
+    (128, 1024, 4096, False, True), (128, 2048, 1024, False, True), (96, 2048, 2048, False, True),
+    (128, 1536, 2048, False, True), (96, 3072, 512, False, True), (65, 2048, 6144, True, True), (128, 1024, 12288, True, True),
+    # 97 x 2048 x 2048 0.94, 65 x 2048 x 3072 0.87, 65 x 4096 x 1024 8.1 / 8.2, 65 x 6144 x 1024 8.7 / 12.8
+    (97, 2048, 2048, False, False), (65, 2048, 3072, False, False), (65, 4096, 1024, False, False),
+    (65, 6144, 1024, False, False), (128, 3072, 512, False, False), (65, 2560, 6144, True, False),
+    # up to 64 rows there is nothing to choose; from 129 on the tiles (129 x 1024 x 2048 10.5 / 11.9)
+    (64, 1024, 2048, False, False), (129, 1024, 2048, False, False), (1800, 1024, 2048, False, False),
+])
+def test_products_of_65_to_128_rows(M, N, K, split, gemv):
+    fn = _host("_ZN5ember3hip12gemm_by_gemvERK13EmberGemvArgs", ctypes.c_bool, ctypes.c_void_p)
+    g = _gemv_args(M, N, K, True)
+    need = _lib.lib().ember_hip_gemv_workspace_bytes(64, N, K)
+    assert (need > 0) == split
+    g.workspace, g.workspace_bytes = 256, need  # an address that nothing reads
+    assert fn(ctypes.addressof(g)) is gemv
