@@ -36,6 +36,7 @@
 // logits, top-p 0.95: 303 (523); all equal: 485 (1046), most of it in passes
 // whose atomics all go to one bin.
 #include <cstdint>
+#include <type_traits>
 
 #include "device.hpp"
 #include "kernels.hpp"
@@ -104,20 +105,23 @@ __device__ __forceinline__ float scaled(const float *x, int i, float t) { return
 // memory round trip per batch instead of one per element (a 151,936-logit row
 // is 148 elements per thread).
 constexpr int kRowBatch = 16;
-template <class F>
+// In passes that few rows take (a bin of thousands, a tie's ids): the same time there within 1%, and less code, whose
+// fetching the short launches feel (top-k 40, 16 rows of 151,936: with 81 KB of code 29.5 us, with 71 KB 28.9).
+constexpr int kRareBatch = 8;
+template <int B = kRowBatch, class F>
 __device__ __forceinline__ void for_row(const float *x, int V, F f) {
     int i = static_cast<int>(threadIdx.x);
-    for (; i + (kRowBatch - 1) * kSampleThreads < V; i += kRowBatch * kSampleThreads) {
-        float v[kRowBatch];
+    for (; i + (B - 1) * kSampleThreads < V; i += B * kSampleThreads) {
+        float v[B];
 #pragma unroll
-        for (int u = 0; u < kRowBatch; u++) v[u] = x[i + u * kSampleThreads];
+        for (int u = 0; u < B; u++) v[u] = x[i + u * kSampleThreads];
 #pragma unroll
-        for (int u = 0; u < kRowBatch; u++) f(i + u * kSampleThreads, v[u]);
+        for (int u = 0; u < B; u++) f(i + u * kSampleThreads, v[u]);
     }
     for (; i < V; i += kSampleThreads) f(i, x[i]);
 }
 
-__device__ float block_max(float v, SampleLds &sh) {
+__device__ __forceinline__ float block_max(float v, SampleLds &sh) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
     const int wave = static_cast<int>(threadIdx.x) / kWave;
@@ -129,7 +133,7 @@ __device__ float block_max(float v, SampleLds &sh) {
     return m;
 }
 
-__device__ unsigned long long block_sum_u64(unsigned long long v, SampleLds &sh) {
+__device__ __forceinline__ unsigned long long block_sum_u64(unsigned long long v, SampleLds &sh) {
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
     const int wave = static_cast<int>(threadIdx.x) / kWave;
@@ -142,7 +146,7 @@ __device__ unsigned long long block_sum_u64(unsigned long long v, SampleLds &sh)
 }
 
 // The sum of v over the threads before this one (and, in total, over all).
-__device__ unsigned long long block_scan_u64(unsigned long long v, SampleLds &sh, unsigned long long &total) {
+__device__ __forceinline__ unsigned long long block_scan_u64(unsigned long long v, SampleLds &sh, unsigned long long &total) {
     const int lane = static_cast<int>(threadIdx.x) % kWave, wave = static_cast<int>(threadIdx.x) / kWave;
     unsigned long long incl = v;
 #pragma unroll
@@ -187,26 +191,35 @@ __device__ __forceinline__ void sort_list(int n, SampleLds &sh) {
     __syncthreads();
     for (int i = n + tid; i < size; i += kSampleThreads) sh.list[i] = 0;
     __syncthreads();
-    // Up to j = 64 a wave's pairs lie within its own 128 entries, and its LDS operations run in order: a barrier only
-    // before and after steps that reach further. (One after each of the 66 steps of 2048 entries: 3 us more.)
-    for (int k = 2; k <= size; k *= 2)
-        for (int j = k / 2; j > 0; j /= 2) {
-            if (tid < size / 2) {  // pair (i, i + j); kList / 2 threads at most
-                const int i = 2 * tid - (tid & (j - 1));
-                const unsigned long long a = sh.list[i], b = sh.list[i + j];
-                if (((i & k) == 0) == (a < b)) {
-                    sh.list[i] = b;
-                    sh.list[i + j] = a;
-                }
-            }
-            const int next = j > 1 ? j / 2 : k;
-            if (max(j, next) > kWave) {
-                __syncthreads();
-            } else {
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-                __builtin_amdgcn_wave_barrier();
+    // Up to j = 64 a wave's pairs lie within its own 128 entries, and its LDS operations run in order: those steps need no
+    // barrier, and waves without entries no part in them. (A barrier after each of the 66 steps of 2048 entries: 3 us more.)
+    auto step = [&](int k, int j) {
+        if (tid < size / 2) {  // pair (i, i + j); kList / 2 threads at most
+            const int i = 2 * tid - (tid & (j - 1));
+            const unsigned long long a = sh.list[i], b = sh.list[i + j];
+            if (((i & k) == 0) == (a < b)) {
+                sh.list[i] = b;
+                sh.list[i + j] = a;
             }
         }
+    };
+    auto narrow = [&](int k, int j) {
+        if (tid - tid % kWave >= size / 2) return;
+        for (; j > 0; j /= 2) {
+            step(k, j);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    for (int k = 2; k <= min(size, 2 * kWave); k *= 2) narrow(k, k / 2);
+    for (int k = 4 * kWave; k <= size; k *= 2) {
+        __syncthreads();
+        for (int j = k / 2; j > kWave; j /= 2) {
+            step(k, j);
+            __syncthreads();
+        }
+        narrow(k, kWave);
+    }
     __syncthreads();
 }
 
@@ -239,11 +252,11 @@ __device__ __forceinline__ int block_first_largest(float best, int idx, SampleLd
 }
 
 // First largest score(i, x[i]) over i < V (ties to the lowest index).
-template <class F>
+template <int B = kRowBatch, class F>
 __device__ __forceinline__ int block_argmax(const float *x, int V, F score, SampleLds &sh) {
     float best = -INFINITY;
     int idx = 0x7fffffff;
-    for_row(x, V, [&](int i, float xi) {
+    for_row<B>(x, V, [&](int i, float xi) {
         const float v = score(i, xi);
         if (v > best) {  // i ascends per thread: the first of equal values is kept
             best = v;
@@ -268,7 +281,7 @@ __device__ __forceinline__ int kth_tied_id(const float *x, int V, float t, const
         for (int i = tid; i < 256; i += kSampleThreads) sh.hist[i] = 0;
         __syncthreads();
         const uint32_t prefix = sh.prefix, mask = sh.mask;
-        for_row(x, V, [&](int i, float xi) {
+        for_row<kRareBatch>(x, V, [&](int i, float xi) {
             const float v = xi / t;
             if (v != theta || !within.keeps(v, i) || (static_cast<uint32_t>(i) & mask) != prefix) return;
             atomicAdd(&sh.hist[(static_cast<uint32_t>(i) >> shift) & 255u], 1ull);
@@ -334,13 +347,15 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
                                           float top_p, unsigned long long &kept, SampleLds &sh) {
     const int tid = static_cast<int>(threadIdx.x);
     const bool prob = top_p >= 0.0f;
+    using Batch = std::integral_constant<int, kRowBatch>;
+    using Rare = std::integral_constant<int, kRareBatch>;
     auto weight = [&](float v) { return prob ? fixed_weight(v, mx) : 1ull; };
     // The sums of bin_of(v)'s bins over the elements of `within` above -inf (bin < 0: left out).
-    auto fill_bins = [&](auto bin_of) {
+    auto fill_bins = [&](auto batch, auto bin_of) {
         __syncthreads();
         for (int i = tid; i < kBins; i += kSampleThreads) sh.bins[i] = 0;
         __syncthreads();
-        for_row(x, V, [&](int i, float xi) {
+        for_row<decltype(batch)::value>(x, V, [&](int i, float xi) {
             const float v = xi / t;
             if (!(v > -INFINITY)) return;
             const int b = bin_of(v);
@@ -353,7 +368,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
     // The elements of `within` above -inf that in(v) takes, into sh.list: how many they are and, where the list does not
     // hold them, their lowest and highest key.
     uint32_t low = 0, high = 0;
-    auto collect = [&](auto in) {
+    auto collect = [&](auto batch, auto in) {
         if (tid == 0) {
             sh.listed = 0;
             sh.low = ~0u;
@@ -362,7 +377,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
         __syncthreads();
         low = ~0u;
         high = 0;
-        for_row(x, V, [&](int i, float xi) {
+        for_row<decltype(batch)::value>(x, V, [&](int i, float xi) {
             const float v = xi / t;
             if (!(v > -INFINITY) || !in(v) || !within.keeps(v, i)) return;
             const int at = atomicAdd(&sh.listed, 1);
@@ -394,7 +409,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
         const float d = (mx - v) * kBinsPerUnit;
         return d < static_cast<float>(kBins - 1) ? static_cast<int>(d) : kBins - 1;
     };
-    fill_bins(step_of);
+    fill_bins(Batch{}, step_of);
     unsigned long long target = 0;
     auto set_target = [&](unsigned long long total) {
         return target = prob ? top_p_target(top_p, total) : static_cast<unsigned long long>(top_k);
@@ -402,12 +417,12 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
     if (!find_bin(0, set_target, kept, sh)) return within;
     const int step = static_cast<int>(sh.prefix);
     unsigned long long above = sh.above;
-    int n = collect([&](float v) { return step_of(v) == step; });
+    int n = collect(Batch{}, [&](float v) { return step_of(v) == step; });
 #pragma unroll 1
     while (n > kList && low < high) {  // at most three times: 32 bits of key, 11 of them a time
         const int shift = max(0, 32 - __clz(static_cast<int>(high - low)) - 11);  // (high - low) >> shift < kBins
         const uint32_t lo = low, hi = high;
-        fill_bins([&](float v) {
+        fill_bins(Rare{}, [&](float v) {
             const uint32_t k = order_key(v) - lo;
             return k > hi - lo ? -1 : kBins - 1 - static_cast<int>(k >> shift);
         });
@@ -416,7 +431,7 @@ __device__ __forceinline__ Cut prefix_cut(const float *x, int V, float t, const 
         const uint32_t part = static_cast<uint32_t>(kBins - 1) - sh.prefix;
         above = sh.above;
         __syncthreads();  // every thread has read sh before it is reused
-        n = collect([&](float v) {
+        n = collect(Rare{}, [&](float v) {
             const uint32_t k = order_key(v) - lo;
             return k <= hi - lo && k >> shift == part;
         });
@@ -600,7 +615,7 @@ __global__ void __launch_bounds__(kSampleThreads) sample_kernel(const float *__r
     if (d.greedy) {
         tok = block_argmax(x, V, [](int, float xi) { return xi; }, sh);
     } else if (d.certain) {
-        tok = block_argmax(x, V, [&](int, float xi) { return xi / d.t; }, sh);
+        tok = block_argmax<kRareBatch>(x, V, [&](int, float xi) { return xi / d.t; }, sh);
     } else if (d.listed) {
         float best = -INFINITY;
         int idx = 0x7fffffff;
@@ -641,7 +656,7 @@ __global__ void __launch_bounds__(kSampleThreads) prob_kernel(const float *__res
     if (d.greedy) {
         prob = block_argmax(x, V, [](int, float xi) { return xi; }, sh) == tok ? 1.0f : 0.0f;
     } else if (d.certain) {  // 0 for every token of a row with nothing above -inf
-        prob = block_argmax(x, V, [&](int, float xi) { return xi / d.t; }, sh) == tok && d.mx > 0.0f ? 1.0f : 0.0f;
+        prob = block_argmax<kRareBatch>(x, V, [&](int, float xi) { return xi / d.t; }, sh) == tok && d.mx > 0.0f ? 1.0f : 0.0f;
     } else {
         const float v = scaled(x, tok, d.t);
         const float w = expf(v - d.mx);
