@@ -11,13 +11,14 @@
 // reads it. A comes in chunks of two k steps, double-buffered, its loads two
 // chunks ahead in registers; W's loads run two chunks ahead too. Taking a run's
 // strided steps one at a time would read A in 64-byte pieces (1800 x 4096 x
-// 1024 29.1 us); two runs side by side read 128.
+// 1024 29.1 us against 26.4, weights in the last-level cache); two runs side by
+// side read 128.
 //
-// Measured (packed W, a graph of 60 launches over 8 weights), against 64 rows
-// per launch of the decode-sized kernel: 1800 x 4096 x 1024 26.4 us (572
-// TFLOP/s), 129 before; 1800 x 1024 x 2048 17.9, 121; 1800 x 6144 x 1024 40.8,
-// 229; 1800 x 1024 x 3072 22.9, 163; 256 x 4096 x 1024 7.7, 19.1; 256 x 1024 x
-// 2048 9.4, 16.8; 48 x 12288 x 2048 15.4, 27.3; 64 x 151936 x 1024 72, 135.
+// Measured, packed W from HBM, against 64 rows per launch of the decode-sized
+// kernel (us): 1800 x 4096 x 1024 29 (520 TFLOP/s), 128 before; 1800 x 1024 x 2048
+// 18.8, 120; 1800 x 6144 x 1024 44, 229; 1800 x 1024 x 3072 26, 162; 256 x 4096 x 1024
+// 8.7, 18.6; 256 x 1024 x 2048 11.7, 16.4; 48 x 12288 x 2048 16.3, 27.6; 64 x 151936 x
+// 1024 76, 147.
 #include <algorithm>
 #include <type_traits>
 
@@ -405,20 +406,21 @@ bool gemm_by_gemv(const EmberGemvArgs &a) {
     return a.N <= 3072 && a.K <= 512 && a.M <= 96;
 }
 
-// The form by the number of work-groups (us; packed W):
+// The form by the number of work-groups (us; packed W from HBM):
 //  - the split form while its 64 x 64 blocks fit one round at one per CU: its
-//    waves each walk a quarter of K (256 x 1024 x 2048, 64 work-groups, 9.4
-//    against 12.2 with one feature tile per wave and 15.8 with two; 256 x 4096 x
-//    1024, 256, 7.7 / 8.4 / 10.2; 256 x 6144 x 1024, 384, 13.3 / 10.5 / 11.1).
+//    waves each walk a quarter of K (256 x 1024 x 2048, 64 work-groups, 11.7
+//    against 13.1 with one feature tile per wave and 16.3 with two; 256 x 4096 x
+//    1024, 256, 8.7 / 9.0 / 10.7; 256 x 6144 x 1024, 384, 14.5 / 11.3 / 11.8).
 //    Its LDS reads, 64 rows per feature tile, bound it beyond;
 //  - two feature tiles per wave, which read A half as often, from 200
-//    work-groups on (1800 x 6144 x 1024, one against two, 42.6 / 40.8; 1800 x
-//    1024 x 2048, 232 work-groups, 18.4 / 17.9); up to 64 rows, where W's one
-//    pass is what counts, one (64 x 151936 x 1024 71.8 / 76.6);
+//    work-groups on (1800 x 12288 x 2048, one against two, 169 / 142; 1800 x 1024 x
+//    2048, 232 work-groups, 19.2 / 18.8; 700 x 2048 x 2048, 176, 17.8 / 18.4); up to 64
+//    rows, where W's one pass is what counts, one (64 x 151936 x 1024 75.9 / 78);
 //  - else one. Four feature tiles spilled and were within 2% of two; 128 tokens
-//    per work-group, at one wave per SIMD, lost (1800 x 4096 x 1024 34.3 / 27.1).
-// A row-major W's split form is slower than one tile per wave (48 x 6144 x 2048
-// 14.3 / 12.7).
+//    per work-group, at one wave per SIMD, lost (1800 x 4096 x 1024 34.3 / 27.1,
+//    weights in the last-level cache).
+// A row-major W's split form is no faster than one tile per wave (48 x 6144 x
+// 2048 16.5 / 16.4).
 hipError_t launch_gemm(const EmberGemvArgs &a, hipStream_t stream) {
     const int m_blocks = (a.M + 63) / 64;
     const int ks = slices(a);
