@@ -16,7 +16,8 @@
 //     ember_hip_token_probs), logits copied out on request.
 // Every launch goes to one stream of default priority. The linear layers of
 // steps beyond the decode-sized GEMV's 64 rows (prompt chunks) run on the tiled
-// kernel (gemm.hip), which gives each row the GEMV's bits.
+// kernel (gemm.hip), which gives each row the GEMV's bits; up to 128 rows, those
+// of few features run 64 rows at a time.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

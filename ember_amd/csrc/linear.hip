@@ -86,7 +86,8 @@ constexpr int kNormFused = 2048;  // and their width at most
 // MT tiles of 16 tokens (M <= 16 MT); EP an EMBER_EPILOGUE_*; SPLIT: K split
 // over gridDim.y work-groups (a separate instance, so the unsplit one keeps
 // its constant-stride loads and no merge code). Dynamic LDS: the staged
-// activations (staged) or nothing, and afterwards the waves' partial sums.
+// activations (staged), the waves' own stages (a split launch that stages none)
+// or nothing, and afterwards the waves' partial sums.
 // NORM: A is the f32 residual, lda its row length, and the staged activations
 // are its RMSNorm (rmsnorm_rows_kernel's arithmetic in its order, so its bits),
 // computed by every work-group for itself: up to kNormRows rows are a few KiB,

@@ -665,9 +665,9 @@ def test_gemv_matches_oracle(device, M, N, KD, ep, split):
 @pytest.mark.parametrize("N,KD", [(4096, 2048), (2048, 2048), (2048, 6144), (1024, 3072)])
 @pytest.mark.parametrize("ep", [0, 2])
 def test_gemv_rows_do_not_depend_on_the_batch(device, N, KD, ep):
-    """A token's outputs are the same bits whatever the batch around it. The batches here take both activation
-    paths: up to 32 rows of a 2048-wide K slice (16 of a 3072-wide one) are staged in LDS, more rows are read
-    straight from A. With fewer than 256 feature blocks (2048 and 1024 features) a batch of more than 16 tokens
+    """A token's outputs are the same bits whatever the batch around it. The batches here take every activation
+    path: up to 32 rows of a 2048-wide K slice (16 of a 3072-wide one) are staged in LDS, more rows are read
+    straight from A, or, split, through each wave's own stage. With fewer than 256 feature blocks (2048 and 1024 features) a batch of more than 16 tokens
     runs one 16-token tile per work-group. The split shape (2048 x 6144 over 2 slices) goes through the merge."""
     from ember_amd import _lib
     rng = np.random.default_rng(N + KD + ep)
@@ -892,9 +892,10 @@ def test_gemv_rows_gigabytes_apart(device, M, N, KD, split):
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("ep", [0, 1, 2, 3])
 def test_gemv_batches_on_tiles_equal_16_rows_at_a_time(device, M, N, KD, packed, ep):
-    """Batches of 17 to 64 tokens whose activations are too large to stage (33 and 64 rows), or whose packed W is large,
-    go to the tiled kernel: the same bits as 16 rows at a time, for both W layouts, ragged features, steps that do not
-    divide into the runs (1376: 43; 288: 9), and more blocks than one round. 4096 features stay with the GEMV."""
+    """Batches of 17 to 64 tokens whose packed W is large go to the tiled kernel: the same bits as 16 rows at a time, for
+    ragged features, steps that do not divide into the runs (288: 9), and more blocks than one round. Row-major W, 4096
+    features, and activations too large to stage whose rows are not whole 128-byte lines (1376, 2080) stay with the
+    GEMV."""
     from ember_amd import _lib
     rng = np.random.default_rng(M + N + KD + ep)
     a = torch.from_numpy(rng.standard_normal((M, KD)).astype(np.float16)).to(device)

@@ -165,8 +165,8 @@ def _row(kind, V, rng):
 @pytest.mark.parametrize("kind", ["flat", "peaked", "tied", "masked"])
 @pytest.mark.parametrize("V", [40, 1023, 4999, 151936])
 def test_every_way_to_the_cuts_keeps_the_hosts_set(kind, V):
-    """Top-k from the threads' maxima (k 1 to 512), through bins (beyond) and by radix (bins with more ties than the
-    list), top-p alone and inside top-k, min-p alone and after them: the draws are the host sampler's, and the tokens
+    """Top-k from the threads' maxima (k up to 512; in short rows up to V / 32, 128 at least), through bins (beyond), and
+    through bins with more elements than the list, top-p alone and inside top-k, min-p alone and after them: the draws are the host sampler's, and the tokens
     either side of the cut have the host's probabilities (the first left out: 0)."""
     rng = np.random.default_rng(V + len(kind))
     x = _row(kind, V, rng)
@@ -188,7 +188,7 @@ def test_every_way_to_the_cuts_keeps_the_hosts_set(kind, V):
 
 
 def test_rows_with_infinities_and_nan():
-    """A NaN logit is never drawn, as if it were -inf."""
+    """A NaN logit is never drawn, as if it were -inf; a row of -inf draws token 0. (+inf: the test below.)"""
     rng = np.random.default_rng(3)
     x = rng.normal(0.0, 2.0, 5000).astype(np.float32)
     clean = x.copy()
